@@ -288,6 +288,20 @@ size_t exl3_gemm_trellis_workspace_size(int m, int k, const int* widths, int gro
  * Callers: exl3rocm's prefill workspace. */
 size_t exl3_gemm_trellis_workspace_bound(void);
 
+/* The workspace with which exl3_gemm_trellis_grouped and exl3_gemm_trellis_silu_in take their fastest
+ * plan for every shape: exl3_gemm_trellis_workspace_bound() bytes (split prefill tiles, or the
+ * register-decode GEMM's partial tiles, up to 128 rows), then that GEMM's completion counters.  Zero
+ * before the first call; every call leaves its counters zero.  With a smaller workspace up to 128
+ * rows take the prefill GEMM: the same results to the tolerance.  No reference counterpart.
+ * Callers: exl3rocm's prefill workspace. */
+size_t exl3_gemm_trellis_workspace_max(void);
+
+/* Self-check of the register-decode GEMM's unit split for a launch (host only, no GPU): the kernel's
+ * 32-bit division forms against brute force.  Returns the number of mismatches (0), or -1 for a shape
+ * that GEMM does not serve (more than 128 rows, k below 2048 or not a multiple of 256).  No
+ * reference counterpart.  Callers: the CPU tests. */
+int exl3_gemm_rd_check(int m, int k, const int* widths, int groups);
+
 /* Dispatcher by row count: m <= 32 -> fused GEMV, else the prefill GEMM.  Returns the route
  * tag (1 = GEMV, 2 = prefill GEMM) or a negative error.
  * Replaces `exl3_gemm(A, B, C, suh, A_had, svh, -1, mcg, mul1, 0) -> int` (reference ops.py:82). */

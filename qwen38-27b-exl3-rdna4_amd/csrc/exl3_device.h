@@ -20,6 +20,8 @@
 #include <stdint.h>
 #include "../../include/exl3_mi355x.h"
 
+#include <utility>
+
 namespace exl3 {
 
 typedef _Float16 f16;
@@ -28,6 +30,38 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// f(integral_constant<int, I>) for I in the sequence: ring slots are indexed by constants in the
+// source, so a ring always lives in registers (a loop index there could leave it in scratch memory)
+template <class F, int... I>
+__device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&& f)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+// n / d for 32-bit unsigned n and an invariant divisor d >= 1 in a multiply-high, a subtract and
+// two shifts (Granlund and Montgomery, "Division by invariant integers using multiplication",
+// PLDI 1994, figure 4.1): m = floor(2^32 (2^l - d) / d) + 1 with l = ceil(log2 d).  The unit
+// split's divisions run on the completion path of every launch; 64-bit divisions there cost
+// hundreds of instructions each.
+struct UDiv {
+    uint32_t m, s1, s2;
+    static UDiv of(uint32_t d)
+    {
+        int l = 0;
+        while ((1ull << l) < d) ++l;
+        UDiv r;
+        r.m = (uint32_t) (((1ull << 32) * ((1ull << l) - d)) / d + 1);
+        r.s1 = l > 0 ? 1u : 0u;
+        r.s2 = l > 0 ? (uint32_t) (l - 1) : 0u;
+        return r;
+    }
+    __host__ __device__ uint32_t div(uint32_t n) const
+    {
+        const uint32_t t = (uint32_t) (((uint64_t) m * n) >> 32);
+        return (t + ((n - t) >> s1)) >> s2;
+    }
+};
 
 constexpr double R_SCALE = 0.088388347648;   // the Hadamard scale of every reference call site
 
@@ -358,6 +392,17 @@ __device__ __forceinline__ uint32_t silu_mul_x2(uint32_t g, uint32_t u)
         r[i] = (f16) ((float) act * (float) uh[i]);
     }
     return __builtin_bit_cast(uint32_t, r);
+}
+
+// Fragment order of a rotated input [rows][cols] (the register-decode GEMM's, v_mfma_f32_32x32x16_f16
+// operands as contiguous loads): row tiles of 32 rows (the last one: its live rows only), in each the
+// 32-column slices, in each the 8-column parts in the order (column bit 3, column bit 4), in each
+// the rows' 8 halves.  Offset (halves) of element (row, col).
+__device__ __forceinline__ int64_t frag_offset(int row, int col, int rows, int cols)
+{
+    const int T = row >> 5, n = min(32, rows - 32 * T);
+    return (int64_t) T * 32 * cols + (int64_t) (col >> 5) * n * 32 +
+           ((((col >> 3) & 1) * 2 + ((col >> 4) & 1)) * n + (row & 31)) * 8 + (col & 7);
 }
 
 // the (pre, out) pair of each group of one launch (a fused module's input transforms read one x)

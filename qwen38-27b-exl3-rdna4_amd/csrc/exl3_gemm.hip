@@ -13,6 +13,7 @@
 // exl3_hgemm_recon is the same GEMM with a dense fp16 W[k, n] as the B source and a plain
 // fp16 C epilogue.
 #include "exl3_device.h"
+#include "exl3_gemm_rd.h"
 #include "../../include/exl3_mi355x.h"
 
 #include <stdlib.h>
@@ -23,7 +24,7 @@ using namespace exl3;
 
 // had_r_128 of one input into several outputs in one launch (exl3_gemv.hip)
 int launch_had(const void* in, int64_t ld_in, void* const* out, int64_t ld_out, int rows, int cols, const void* const* pre,
-               int groups, const void* post, float scale, void* stream, bool exact, const void* in_up);
+               int groups, const void* post, float scale, void* stream, bool exact, const void* in_up, bool fragments = false);
 
 namespace {
 
@@ -836,10 +837,22 @@ int gemm_trellis_common(const void* x, int64_t ldx, const void* const* trellis, 
         xhs[i] = xi;
         svs[i] = (const uint16_t*) svh[i];
     }
-    // the groups' input transforms (one x, each group's suh) in one launch
-    const int rc = launch_had(x, ldx, xo, k, m, k, suh, groups, nullptr, 1.0f, s, false, x_up);
-    if (rc) return rc;
     const int cb = codebook_of(mcg, mul1);
+    // up to 128 rows the register-decode GEMM (exl3_gemm_rd.hip; its plan says which shapes): its partial
+    // tiles in the prefill's, its counters behind them.  EXL3_GEMM_KERNEL set (comparisons): not taken.
+    const char* e = getenv("EXL3_GEMM_KERNEL");
+    RdPlan rd{};
+    if (ws && wsb >= exl3_gemm_trellis_workspace_max() && !(e && e[0])) rd = rd_plan(m, k, widths, groups);
+    bool use_rd = rd.use && rd.part_bytes <= exl3_gemm_trellis_workspace_bound() - PC_COUNTER_BYTES &&
+                  (uint64_t) m * (uint64_t) ldy * 2 < (1ull << 31);
+    for (int i = 0; i < groups; ++i) use_rd = use_rd && (uint64_t) k * widths[i] * K / 8 < (1ull << 31);
+    // the groups' input transforms (one x, each group's suh) in one launch: the float32 sums of the
+    // prefill; the GEMV's exact ones for the register-decode GEMM up to the GEMV's 64 rows
+    const int rc = launch_had(x, ldx, xo, k, m, k, suh, groups, nullptr, 1.0f, s, use_rd && m <= EXL3_GEMV_MAX_ROWS, x_up, use_rd);
+    if (rc) return rc;
+    if (use_rd)
+        return launch_gemm_rd(rd, K, cb, xhs, trellis, y, ldy, svs, widths, groups, m, k, (char*) ws + PC_COUNTER_BYTES,
+                              (uint32_t*) ((char*) ws + exl3_gemm_trellis_workspace_bound()), s);
     switch (K) {
         case 1: return launch_trellis_gemm_cb<1>(cb, xhs, k, trellis, y, ldy, svs, widths, groups, m, k, ws, wsb, s);
         case 2: return launch_trellis_gemm_cb<2>(cb, xhs, k, trellis, y, ldy, svs, widths, groups, m, k, ws, wsb, s);
@@ -895,6 +908,11 @@ size_t exl3_gemm_trellis_workspace_bound(void)
     // pieces of one plan: full >= 1 or 2 tail <= CUs: tail * min(CUs / tail, .) <= CUs; the
     // two-piece form: 2 tail with 3 tail <= 2 CUs
     return PC_COUNTER_BYTES + (size_t) std::max(PC_CUS, 2 * (2 * PC_CUS / 3)) * PC_PIECE_BYTES;
+}
+
+size_t exl3_gemm_trellis_workspace_max(void)
+{
+    return exl3_gemm_trellis_workspace_bound() + (size_t) RD_MAX_TILES * sizeof(uint32_t);
 }
 
 int exl3_gemm_trellis_grouped(const void* x, int64_t ldx, const void* const* trellis, void* y, int64_t ldy,

@@ -143,7 +143,8 @@ __global__ void __launch_bounds__(256) had_kernel(const uint16_t* __restrict__ i
 // same values bit for bit: both sum exactly in float64 and round once (scaled_f16), with the
 // same fp16 products for pre, post and the SiLU input.  A wave reads its whole block before any
 // lane writes, so in == out is safe.
-template <class T>
+// FRAG: the outputs in the fragment order of the register-decode GEMM (frag_offset), ld_out unused.
+template <class T, bool FRAG>
 __global__ void __launch_bounds__(256) had_kernel_x2(const uint16_t* __restrict__ in, const uint16_t* __restrict__ in_up,
                                                      int64_t ld_in, HadGroups hg, int groups, int64_t ld_out, int rows,
                                                      int cols, const uint16_t* __restrict__ post, T scale)
@@ -157,25 +158,26 @@ __global__ void __launch_bounds__(256) had_kernel_x2(const uint16_t* __restrict_
     uint32_t v = *reinterpret_cast<const uint32_t*>(in + row * ld_in + col);
     if (in_up) v = silu_mul_x2(v, *reinterpret_cast<const uint32_t*>(in_up + row * ld_in + col));
     const uint32_t q = post ? *reinterpret_cast<const uint32_t*>(post + col) : 0u;
+    const int64_t o = FRAG ? frag_offset((int) row, col, rows, cols) : row * ld_out + col;
     for (int g = 0; g < groups; ++g) {
         // constant indices into the argument struct (a runtime index would copy it to scratch)
         const uint16_t* pre = g == 0 ? hg.pre[0] : g == 1 ? hg.pre[1] : g == 2 ? hg.pre[2] : hg.pre[3];
         uint16_t* out = g == 0 ? hg.out[0] : g == 1 ? hg.out[1] : g == 2 ? hg.out[2] : hg.out[3];
         const uint32_t p = pre ? *reinterpret_cast<const uint32_t*>(pre + col) : 0u;
-        *reinterpret_cast<uint32_t*>(out + row * ld_out + col) = had128_x2<T>(v, p, pre != nullptr, q, post != nullptr, scale);
+        *reinterpret_cast<uint32_t*>(out + o) = had128_x2<T>(v, p, pre != nullptr, q, post != nullptr, scale);
     }
 }
 
 // the float transform's launch (exl3_had.hip)
 void launch_had_mfma(const uint16_t* in, const uint16_t* up, int64_t ld_in, const HadGroups& hg, int groups,
-                     int64_t ld_out, int rows, int cols, const uint16_t* post, float scale, bool has_pre, hipStream_t s);
+                     int64_t ld_out, int rows, int cols, const uint16_t* post, float scale, bool has_pre, bool fragments, hipStream_t s);
 
 // had_r_128 of one input into `groups` outputs, group i scaled by pre[i] (may be null; the float32
 // form takes a pre for every group or for none): one launch (the prefill's input transforms of a
 // fused module); exact: float64 butterflies, else float32 sums on the matrix cores (the prefill's
 // input transforms and epilogue values)
 int launch_had(const void* in, int64_t ld_in, void* const* out, int64_t ld_out, int rows, int cols, const void* const* pre,
-               int groups, const void* post, float scale, void* stream, bool exact, const void* in_up)
+               int groups, const void* post, float scale, void* stream, bool exact, const void* in_up, bool fragments)
 {
     if (((uintptr_t) in_up) & 15) return EXL3_EINVAL;
     if (!in || !out || rows < 0 || cols % 128 || cols < 128 || ld_in < cols || ld_out < cols || ld_in % 8 || ld_out % 8 ||
@@ -189,6 +191,7 @@ int launch_had(const void* in, int64_t ld_in, void* const* out, int64_t ld_out, 
         hg.out[i] = (uint16_t*) out[i];
     }
     if (rows == 0) return EXL3_OK;
+    if (fragments && exact && rows > EXL3_GEMV_MAX_ROWS) return EXL3_EINVAL;
     const int64_t jobs = (int64_t) rows * (cols / 128);           // 8 lanes each
     const dim3 grid((unsigned) ((jobs + 31) / 32));
     if (!exact) {
@@ -198,12 +201,13 @@ int launch_had(const void* in, int64_t ld_in, void* const* out, int64_t ld_out, 
         int n_pre = 0;
         for (int i = 0; i < groups; ++i) n_pre += hg.pre[i] != nullptr;
         if (n_pre != 0 && n_pre != groups) return EXL3_EINVAL;      // pre for every group or for none
+        if (fragments && (n_pre != groups || post)) return EXL3_EINVAL;
         launch_had_mfma((const uint16_t*) in, (const uint16_t*) in_up, ld_in, hg, groups, ld_out, rows, cols,
-                        (const uint16_t*) post, sc, n_pre != 0, (hipStream_t) stream);
+                        (const uint16_t*) post, sc, n_pre != 0, fragments, (hipStream_t) stream);
     } else if (rows <= EXL3_GEMV_MAX_ROWS) {
         // the latency form: one block per wave, four waves a workgroup
-        hipLaunchKernelGGL(had_kernel_x2<double>, dim3((unsigned) ((jobs + 3) / 4)), dim3(256), 0, (hipStream_t) stream,
-                           (const uint16_t*) in, (const uint16_t*) in_up, ld_in, hg, groups, ld_out, rows, cols,
+        hipLaunchKernelGGL((fragments ? had_kernel_x2<double, true> : had_kernel_x2<double, false>),
+                           dim3((unsigned) ((jobs + 3) / 4)), dim3(256), 0, (hipStream_t) stream, (const uint16_t*) in, (const uint16_t*) in_up, ld_in, hg, groups, ld_out, rows, cols,
                            (const uint16_t*) post, R_SCALE * (double) scale);
     } else {
         hipLaunchKernelGGL(had_kernel<double>, grid, dim3(256), 0, (hipStream_t) stream, (const uint16_t*) in,
@@ -459,7 +463,7 @@ int gemv_common(const void* x, int64_t ldx, const GemvGroup* gs, const int* widt
             outs[i] = (uint16_t*) xr + (int64_t) i * m * k;
             pres[i] = gs[i].suh;
         }
-        const int rc = launch_had(x, ldx, outs, k, m, k, pres, groups, nullptr, 1.0f, stream, true, x_up);
+        const int rc = launch_had(x, ldx, outs, k, m, k, pres, groups, nullptr, 1.0f, stream, true, x_up, false);
         if (rc != EXL3_OK) return rc;
         a.xr = (const uint16_t*) xr;
         a.x_up = nullptr;                       // the activation is in the pre-rotated rows
@@ -778,7 +782,7 @@ int exl3_had_r_128(const void* in, int64_t ld_in, void* out, int64_t ld_out, int
 {
     void* const outs[1] = {out};
     const void* const pres[1] = {pre};
-    return launch_had(in, ld_in, outs, ld_out, rows, cols, pres, 1, post, scale, stream, true, nullptr);
+    return launch_had(in, ld_in, outs, ld_out, rows, cols, pres, 1, post, scale, stream, true, nullptr, false);
 }
 
 int exl3_had_r_128_f32(const void* in, int64_t ld_in, void* out, int64_t ld_out, int rows, int cols, const void* pre,
@@ -786,7 +790,7 @@ int exl3_had_r_128_f32(const void* in, int64_t ld_in, void* out, int64_t ld_out,
 {
     void* const outs[1] = {out};
     const void* const pres[1] = {pre};
-    return launch_had(in, ld_in, outs, ld_out, rows, cols, pres, 1, post, scale, stream, false, nullptr);
+    return launch_had(in, ld_in, outs, ld_out, rows, cols, pres, 1, post, scale, stream, false, nullptr, false);
 }
 
 }  // extern "C"

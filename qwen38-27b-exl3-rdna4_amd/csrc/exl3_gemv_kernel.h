@@ -5,19 +5,9 @@
 #include "exl3_device.h"
 #include "../../include/exl3_mi355x.h"
 
-#include <utility>
-
 using namespace exl3;
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-// f(integral_constant<int, I>) for I in the sequence: ring slots are indexed by constants in the
-// source, so the ring always lives in registers (a loop index here could leave it in scratch memory)
-template <class F, int... I>
-__device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&& f)
-{
-    (f(std::integral_constant<int, I>{}), ...);
-}
 
 // ============================================================================================
 // Fused GEMV with stream-K balancing
@@ -31,30 +21,6 @@ __device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&&
 // workgroups and the last one sums the partials in workgroup order (fixed for the shape, hence
 // deterministic), rounds C to fp16 and applies the output Hadamard and svh.
 // ============================================================================================
-// n / d for 32-bit unsigned n and an invariant divisor d >= 1 in a multiply-high, a subtract and
-// two shifts (Granlund and Montgomery, "Division by invariant integers using multiplication",
-// PLDI 1994, figure 4.1): m = floor(2^32 (2^l - d) / d) + 1 with l = ceil(log2 d).  The unit
-// split's divisions run on the completion path of every launch; 64-bit divisions there cost
-// hundreds of instructions each.
-struct UDiv {
-    uint32_t m, s1, s2;
-    static UDiv of(uint32_t d)
-    {
-        int l = 0;
-        while ((1ull << l) < d) ++l;
-        UDiv r;
-        r.m = (uint32_t) (((1ull << 32) * ((1ull << l) - d)) / d + 1);
-        r.s1 = l > 0 ? 1u : 0u;
-        r.s2 = l > 0 ? (uint32_t) (l - 1) : 0u;
-        return r;
-    }
-    __host__ __device__ uint32_t div(uint32_t n) const
-    {
-        const uint32_t t = (uint32_t) (((uint64_t) m * n) >> 32);
-        return (t + ((n - t) >> s1)) >> s2;
-    }
-};
-
 struct GemvGroup {
     const uint32_t* trellis;   // tile words
     const uint16_t* suh;

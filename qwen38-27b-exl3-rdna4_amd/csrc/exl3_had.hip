@@ -14,11 +14,12 @@ namespace {
 // has a pre-scale (else none has); POST: post is given.  The loads of x, post and the first group's
 // pre go out together, and each group's pre is requested while the group before it is transformed,
 // so a wave waits for one round trip before its first MFMA (loading each pre-scale piece where it
-// is used had put four dependent round trips per group ahead of the matrix work).  UP: the input
+// is used had put four dependent round trips per group ahead of the matrix work).  FRAG: the outputs in the fragment order of the
+// register-decode GEMM (frag_offset; ld_out unused).  UP: the input
 // rows are fp16(fp16(silu(in)) * up) (a gated MLP's activation, up's rows ld_in apart as in's),
 // formed as they load: the down projection's transform reads gate and up instead of an
 // activation pass's output.  Each wave reads its whole tile before it writes: in place is safe.
-template <bool PRE, bool POST, bool UP>
+template <bool PRE, bool POST, bool UP, bool FRAG>
 __global__ void __launch_bounds__(256) had_mfma_kernel(const uint16_t* __restrict__ in, const uint16_t* __restrict__ up,
                                                        int64_t ld_in, HadGroups hg, int groups, int64_t ld_out, int rows,
                                                        int cols, const uint16_t* __restrict__ post, float scale)
@@ -33,6 +34,8 @@ __global__ void __launch_bounds__(256) had_mfma_kernel(const uint16_t* __restric
     const int col0 = (int) (wid - rg * nblk) * 128 + 8 * g;   // this lane's first column
     const int64_t row = (int64_t) rg * 16 + j;
     const bool live = row < rows;
+    const int64_t frag0 = frag_offset((int) row, col0, rows, cols);     // FRAG: this lane's part of slice 0
+    const int frows = min(32, rows - (int) row / 32 * 32);
     u32x4 xb[4], pv[4], pn[4];
 #pragma unroll
     for (int s_ = 0; s_ < 4; ++s_) {
@@ -66,7 +69,11 @@ __global__ void __launch_bounds__(256) had_mfma_kernel(const uint16_t* __restric
             for (int s_ = 0; s_ < 4; ++s_) xs[s_] = xb[s_];
         }
         had128_mfma16(A, xs, scale, POST, pv, [&](int p, u32x4 v) __attribute__((always_inline)) {
-            if (live) *reinterpret_cast<g_u32x4*>(as_global(out) + row * ld_out + col0 + 32 * p) = v;
+            if constexpr (FRAG) {
+                if (live) *reinterpret_cast<g_u32x4*>(as_global(out) + frag0 + (int64_t) p * frows * 32) = v;
+            } else {
+                if (live) *reinterpret_cast<g_u32x4*>(as_global(out) + row * ld_out + col0 + 32 * p) = v;
+            }
         });
     }
 }
@@ -77,15 +84,16 @@ __global__ void __launch_bounds__(256) had_mfma_kernel(const uint16_t* __restric
 // the arguments): pre for every group (has_pre) or for none; up (may be null): the input rows are
 // fp16(fp16(silu(in)) * up)
 void launch_had_mfma(const uint16_t* in, const uint16_t* up, int64_t ld_in, const HadGroups& hg, int groups,
-                     int64_t ld_out, int rows, int cols, const uint16_t* post, float scale, bool has_pre, hipStream_t s)
+                     int64_t ld_out, int rows, int cols, const uint16_t* post, float scale, bool has_pre, bool fragments, hipStream_t s)
 {
     const int64_t waves = ((int64_t) rows + 15) / 16 * (cols / 128);
     using K = void (*)(const uint16_t*, const uint16_t*, int64_t, HadGroups, int, int64_t, int, int, const uint16_t*, float);
-    static const K kernels[8] = {had_mfma_kernel<false, false, false>, had_mfma_kernel<false, false, true>,
-                                 had_mfma_kernel<false, true, false>,  had_mfma_kernel<false, true, true>,
-                                 had_mfma_kernel<true, false, false>,  had_mfma_kernel<true, false, true>,
-                                 had_mfma_kernel<true, true, false>,   had_mfma_kernel<true, true, true>};
-    const K kern = kernels[(has_pre ? 4 : 0) + (post ? 2 : 0) + (up ? 1 : 0)];
+    static const K kernels[8] = {had_mfma_kernel<false, false, false, false>, had_mfma_kernel<false, false, true, false>,
+                                 had_mfma_kernel<false, true, false, false>,  had_mfma_kernel<false, true, true, false>,
+                                 had_mfma_kernel<true, false, false, false>,  had_mfma_kernel<true, false, true, false>,
+                                 had_mfma_kernel<true, true, false, false>,   had_mfma_kernel<true, true, true, false>};
+    const K frag[2] = {had_mfma_kernel<true, false, false, true>, had_mfma_kernel<true, false, true, true>};
+    const K kern = fragments ? frag[up ? 1 : 0] : kernels[(has_pre ? 4 : 0) + (post ? 2 : 0) + (up ? 1 : 0)];
     hipLaunchKernelGGL(kern, dim3((unsigned) ((waves + 3) / 4)), dim3(256), 0, s, in, up, ld_in, hg, groups, ld_out,
                        rows, cols, post, scale);
 }

@@ -73,20 +73,20 @@ _pf_bound = None
 
 
 def prefill_workspace_bound() -> int:
-    """Bytes of a prefill split workspace that serves every shape (the library's bound, ~43 MB)."""
+    """Bytes of a prefill workspace with which every shape takes its fastest plan (the library's, ~45 MB)."""
     global _pf_bound
     if _pf_bound is None:
-        _pf_bound = int(L.lib().exl3_gemm_trellis_workspace_bound())
+        _pf_bound = int(L.lib().exl3_gemm_trellis_workspace_max())
     return _pf_bound
 
 
 def prefill_workspace(device: torch.device, nbytes: int, stream: Optional[int] = None) -> Optional[torch.Tensor]:
-    """Zeroed workspace of the prefill GEMM's split tail for the current (or given) stream.  A
-    stream's first call outside graph capture allocates the bound every shape fits in
-    (exl3_gemm_trellis_workspace_bound), so a later capture on that stream splits exactly as
-    eager calls do.  A stream that captures before any eager prefill call has none: its launches
-    run unsplit, and the tail tiles' outputs can differ from the eager split's in the last place
-    (another fp32 summation order)."""
+    """Zeroed workspace of the prefill GEMM's split tail and the register-decode GEMM's partial tiles
+    for the current (or given) stream.  A stream's first call outside graph capture allocates the
+    size every shape fits in (exl3_gemm_trellis_workspace_max), so a later capture on that stream
+    splits exactly as eager calls do.  A stream that captures before any eager prefill call has
+    none: its launches run unsplit, and the split tiles' outputs can differ from the eager ones' in
+    the last place (another fp32 summation order)."""
     if nbytes <= 0:
         return None
     device = torch.device(device)
@@ -373,7 +373,7 @@ def exl3_gemm_trellis_silu_in(gate, up, B, C, suh, xh, svh, K: int, mcg: bool, m
     _need(xh.numel() >= m * k and xh.dtype == torch.float16 and xh.is_contiguous(), "gemm silu_in: xh scratch [m, k] fp16")
     ldx = g2.stride(0) if m > 1 else k
     wa = (C_int * 1)(n)
-    ws = prefill_workspace(gate.device, int(L.lib().exl3_gemm_trellis_workspace_size(m, k, wa, 1)))
+    ws = prefill_workspace(gate.device, prefill_workspace_bound())
     L.check(L.lib().exl3_gemm_trellis_silu_in(g2.data_ptr(), u2.data_ptr(), ldx, B.data_ptr(), C.data_ptr(), _ldy(C, n),
                                               suh.data_ptr(), xh.data_ptr(), svh.data_ptr(), m, k, n, K,
                                               *_cb_flags(mcg, mul1), ws.data_ptr() if ws is not None else None,
@@ -448,7 +448,7 @@ def exl3_gemm_trellis_grouped(A, B: Sequence[torch.Tensor], C, suh: Sequence[tor
     pt, _a = L.ptr_array([b.data_ptr() for b in B])
     ps, _b = L.ptr_array([s.data_ptr() for s in suh])
     pv, _c = L.ptr_array([s.data_ptr() for s in svh])
-    ws = prefill_workspace(A.device, int(L.lib().exl3_gemm_trellis_workspace_size(m, k, wa, g)))
+    ws = prefill_workspace(A.device, prefill_workspace_bound())
     L.check(L.lib().exl3_gemm_trellis_grouped(x2.data_ptr(), x2.stride(0) if m > 1 else k, pt, C.data_ptr(),
                                               _ldy(C, sum(widths)), ps, xh.data_ptr(), pv, wa, g, m, k, K,
                                               *_cb_flags(mcg, mul1), ws.data_ptr() if ws is not None else None,

@@ -11,8 +11,9 @@ or EXL3_MR_MAX rows for every shape when set):
                             equal to the M == 1 call of that row; EXL3_GEMV_APPROX=affine|int8
                             selects the opt-in approximate mul1 forms (unrounded weights, or
                             int8 activations as the reference's EXL3_ROCM_GFX1201_INT8 path)
-  otherwise              -> input Hadamard pass, then the prefill GEMM (trellis decoded into LDS,
-                            fp16 MFMA, fp32 accumulate, output Hadamard and svh in its epilogue);
+  otherwise              -> input Hadamard pass, then a GEMM launch (fp16 MFMA, fp32 accumulate, output
+                            Hadamard and svh in its epilogue): up to 128 rows the register-decode GEMM,
+                            above the prefill GEMM (trellis decoded into LDS);
                             a fused module's groups share one GEMM launch; EXL3_PREFILL=recon takes
                             the reference's reconstruct + hgemm route instead
 """
@@ -31,28 +32,29 @@ def _env_rows(name: str) -> Optional[int]:
     return None if v is None or not v.strip() else min(int(v), _lib.GEMV_MAX_ROWS)
 
 
-# EXL3_MR_MAX (the reference's knob) fixes the GEMV / prefill boundary for every launch; unset, each
-# launch takes the measured crossover of its shape from GEMV_CROSSOVER (shapes outside it: DEFAULT_MR)
+# EXL3_MR_MAX (the reference's knob) fixes the GEMV / GEMM boundary for every launch; unset, each launch
+# takes the measured crossover of its shape from GEMV_CROSSOVER, or for shapes outside it MID_MR where
+# the register-decode GEMM takes over (k a multiple of 256 from MID_K), else DEFAULT_MR
 MR_MAX: Optional[int] = _env_rows("EXL3_MR_MAX")
 DEFAULT_MR = 32
-# Largest row count at which the fused GEMV beats the prefill GEMM, by (k, output columns of the
-# launch: all its groups).  Measured on MI355X for the launches a Qwen3.5-27B checkpoint makes (q/k/v
-# and gate/up grouped as linear_groups groups them, and lm_head): both routes at every M from 2 to
-# 64, graphs of 24 launches over 8 weight copies, 4 bpw, and 2 / 3 bpw where a checkpoint holds them
-# (the boundary moved by <= 4 rows).  Each entry is a boundary b within 1 % of the least summed time
-# over M with no step above 5 % from the GEMV at b rows to the GEMM at b + 1, for every bitrate
-# measured (re-checked for every entry after each change to the GEMV's input rotation; moved only
-# where the old b failed it: 5120 x 5120 15 -> 17, q/k/v 15 -> 19, the k/v pair 33 -> 58; after the
-# one-block-per-wave pre-rotation pass, the 14336-column q/k/v 17 -> 25, 6144 x 5120 32 -> 30 and
-# 17408 x 5120 35 -> 39).  The
-# GEMM's cost is flat within each 16-row MFMA tile; the GEMV's grows with every row and 16-row tile,
-# so the GEMM wins early where its 128-column tiles fill the chip (5120 - 7168 columns: b = 17 - 19)
-# and late where they do not (the k/v launches, 2 x 17408 columns and lm_head: 58 to the GEMV's
-# 64-row limit).
+MID_MR, MID_K = 8, 3072
+# Largest row count at which the fused GEMV beats the GEMM route, by (k, output columns of the launch:
+# all its groups).  Measured on MI355X for the launches a Qwen3.5-27B checkpoint makes (q/k/v and
+# gate/up grouped as linear_groups groups them, and lm_head) and 4096 x 4096: both routes at 20 row
+# counts from 2 to 64, graphs of 16 launches over cold weights, 4 bpw, and 2 / 3 / 5 bpw where a
+# checkpoint holds them.  The GEMV's cost grows with every row, the register-decode GEMM's (up to
+# 128 rows) only with each 32-row tile: they cross at 8 to 9 rows on every shape (5120 -> 5120 14.4 /
+# 15.1 us at 8 rows, 17.4 / 15.1 at 9; gate 25.8 / 24.8 and 27.3 / 24.7; down 24.2 / 25.4 and 26.6 /
+# 25.4; gate/up 38.4 / 37.7 and 39.6 / 37.8), so 8 rows it is: those stay bitwise equal to their
+# one-row calls on every shape.  (lm_head stays at 32: its rows up to there are used as one-row calls'
+# when drafted tokens are verified.)  Up to 8 bpw and for the mcg / 3inst codebooks alike: both routes
+# run the same decoder.  Shapes outside the table: from 3072 inputs the same 8; below them the default
+# 32, the row count up to which a linear has always been its one-row calls (2048 x 2048 16.9 us against
+# 11.1 at 32 rows, 9.0 against 10.7 at 8).
 GEMV_CROSSOVER = {
-    (5120, 1024): 64, (5120, 2048): 58, (5120, 5120): 17, (5120, 6144): 17, (5120, 7168): 19,
-    (5120, 10240): 31, (5120, 12288): 33, (5120, 14336): 25, (5120, 16384): 33, (5120, 17408): 46,
-    (5120, 34816): 64, (5120, 248320): 64, (6144, 5120): 30, (17408, 5120): 39,
+    (5120, 1024): 8, (5120, 2048): 8, (5120, 5120): 8, (5120, 6144): 8, (5120, 7168): 8,
+    (5120, 10240): 8, (5120, 12288): 8, (5120, 14336): 8, (5120, 16384): 8, (5120, 17408): 8,
+    (5120, 34816): 8, (5120, 248320): 32, (6144, 5120): 8, (17408, 5120): 8,
 }
 
 
@@ -60,7 +62,8 @@ def gemv_max_rows(k: int, width: int) -> int:
     """Most rows a launch of k inputs and `width` output columns takes on the fused GEMV."""
     if MR_MAX is not None:
         return MR_MAX
-    return min(GEMV_CROSSOVER.get((k, width), DEFAULT_MR), _lib.GEMV_MAX_ROWS)
+    dflt = MID_MR if k >= MID_K and k % 256 == 0 else DEFAULT_MR
+    return min(GEMV_CROSSOVER.get((k, width), dflt), _lib.GEMV_MAX_ROWS)
 
 
 def gemv_rows(m: int, k: int, width: int) -> bool:
@@ -299,8 +302,8 @@ def exl3_silu_mul_linear(gu: torch.Tensor, trellis: torch.Tensor, suh: torch.Ten
     counterpart in the reference plugin, whose MLP runs a separate SiluAndMul before the down
     linear (the fusion is proposed in reference docs/EFFICIENCY_INVESTIGATION.md:36-66).
 
-    On the GEMV route (<= 32 rows) one GEMV launch forms act from gate and up as its input rows
-    load; on the prefill route the prefill's input transform forms act as it loads the rows (one transform launch and one
+    On the GEMV route one GEMV launch forms act from gate and up as its input rows
+    load; on the GEMM routes the input transform forms act as it loads the rows (one transform launch and one
     GEMM launch, no act in memory); on the approximate GEMV routes and the recon prefill route the
     elementwise kernel writes act and linear runs on it.  Every route equals silu_mul followed by
     linear, bitwise."""
