@@ -137,7 +137,7 @@ def reserve_workspace(device, k: int, n: int, K: int, groups: int = 1, m: Option
 
 def _prep(x: torch.Tensor):
     k = x.shape[-1]
-    x2 = x.reshape(-1, k)
+    x2 = x if x.dim() == 2 and k else x.reshape(-1, k)
     if x2.dtype != torch.float16:
         x2 = x2.to(torch.float16)
     if not x2.is_contiguous():
@@ -179,17 +179,25 @@ def _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y, gemv: Optional[bool] = 
         E.exl3_gemm_trellis_grouped(x2, [trellis], y, [suh], xh, [svh], K, mcg, mul1)
 
 
-@torch.library.custom_op("exl3rocm::linear", mutates_args=())
-def exl3_linear(x: torch.Tensor, trellis: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
-                K: int, mcg: bool, mul1: bool) -> torch.Tensor:
+def _shaped(y: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """The [M, n] result y in the batch shape of x."""
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], y.shape[-1])
+
+
+# The ops' bodies are plain functions: an op whose body needs another's calls that body, not the op
+# (a custom op's way through the dispatcher takes ~7 us of host time, and the outer op has been through it).
+def _linear(x: torch.Tensor, trellis: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
+            K: int, mcg: bool, mul1: bool) -> torch.Tensor:
     x2, k = _prep(x)
     n = svh.shape[0]
     M = x2.shape[0]
     y = torch.empty((M, n), dtype=torch.float16, device=x.device)
-    if M == 0:
-        return y.view(*x.shape[:-1], n)
-    _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y)
-    return y.view(*x.shape[:-1], n)
+    if M:
+        _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y)
+    return _shaped(y, x)
+
+
+exl3_linear = torch.library.custom_op("exl3rocm::linear", mutates_args=())(_linear)
 
 
 @exl3_linear.register_fake
@@ -197,11 +205,10 @@ def _(x, trellis, suh, svh, K, mcg, mul1):
     return x.new_empty((*x.shape[:-1], svh.shape[0]), dtype=torch.float16)
 
 
-@torch.library.custom_op("exl3rocm::linear_groups", mutates_args=())
-def exl3_linear_groups(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch.Tensor],
-                       svh: list[torch.Tensor], K: list[int], mcg: bool, mul1: bool,
-                       ptrs_trellis: Optional[torch.Tensor] = None, ptrs_suh: Optional[torch.Tensor] = None,
-                       ptrs_svh: Optional[torch.Tensor] = None) -> torch.Tensor:
+def _linear_groups(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch.Tensor],
+                   svh: list[torch.Tensor], K: list[int], mcg: bool, mul1: bool,
+                   ptrs_trellis: Optional[torch.Tensor] = None, ptrs_suh: Optional[torch.Tensor] = None,
+                   ptrs_svh: Optional[torch.Tensor] = None) -> torch.Tensor:
     """A fused module made of several checkpoint tensors (e.g. gate_proj + up_proj), each with its
     own K / suh / svh; the concatenation happens inside this opaque op (reference ops.py:106-175).
 
@@ -211,9 +218,9 @@ def exl3_linear_groups(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[t
     kernel, split and output bitwise as exl3_mgemm over the tables), which saves every workgroup a
     dependent load of its table entries before its first trellis request (~1.3 us of a 5120 ->
     2 x 17408 launch)."""
-    widths = [s.shape[0] for s in svh]
     if len(trellis) == 1:
-        return exl3_linear(x, trellis[0], suh[0], svh[0], K[0], mcg, mul1)
+        return _linear(x, trellis[0], suh[0], svh[0], K[0], mcg, mul1)
+    widths = [s.shape[0] for s in svh]
     x2, k = _prep(x)
     M = x2.shape[0]
     ng = len(trellis)
@@ -251,7 +258,10 @@ def exl3_linear_groups(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[t
                                         K[i], mcg, mul1)
         n0 += w
         i = j
-    return y.view(*x.shape[:-1], n0)
+    return _shaped(y, x)
+
+
+exl3_linear_groups = torch.library.custom_op("exl3rocm::linear_groups", mutates_args=())(_linear_groups)
 
 
 @exl3_linear_groups.register_fake
@@ -284,7 +294,7 @@ def exl3_linear_silu_mul(x: torch.Tensor, trellis: list[torch.Tensor], suh: list
     if GATED_ROUTE == "fused" and K[0] == K[1] and fused_rows(M, k, 2 * n):
         E.exl3_gemv_silu_mul(x2, list(trellis), act, list(suh), list(svh), K[0], mcg, mul1)
     else:
-        gu = exl3_linear_groups(x2, trellis, suh, svh, K, mcg, mul1)
+        gu = _linear_groups(x2, trellis, suh, svh, K, mcg, mul1)
         E.silu_mul(gu[:, :n], gu[:, n:], act)
     return act.view(*x.shape[:-1], n)
 

@@ -349,9 +349,13 @@ class Exl3LinearMethod(LinearMethodBase):
         from . import ops  # noqa: F401  (registers the custom ops)
         ng = len(layer.exl3_n)
         per = [[getattr(layer, f"exl3_{kind}_{i}") for i in range(ng)] for kind in TENSOR_KINDS]
-        # one opaque op per module: the groups' outputs are concatenated inside it
-        y = torch.ops.exl3rocm.linear_groups(x, *per, list(layer.exl3_K), layer.exl3_is_mcg, layer.exl3_is_mul1,
-                                             *(layer.exl3_mgemm_ptrs or (None, None, None)))
+        # one opaque op per module: the groups' outputs are concatenated inside it (a module of one tensor
+        # calls linear itself, what linear_groups of one is: its lists cost an eager call 2.5 us)
+        if ng == 1:
+            y = torch.ops.exl3rocm.linear(x, *(p[0] for p in per), layer.exl3_K[0], layer.exl3_is_mcg, layer.exl3_is_mul1)
+        else:
+            y = torch.ops.exl3rocm.linear_groups(x, *per, list(layer.exl3_K), layer.exl3_is_mcg, layer.exl3_is_mul1,
+                                                 *(layer.exl3_mgemm_ptrs or (None, None, None)))
         y = y if y.dtype == x.dtype else y.to(x.dtype)
         return y if bias is None else y + bias
 
