@@ -338,8 +338,8 @@ struct PcArgs {
     int M, K, groups, total, xcd_remap;
     // Balanced tail: items [0, n_full) are whole tiles; every later tile (the last, partial wave of
     // a plain tile grid) is split along K into `split` pieces (split == 1: no split).  A piece
-    // leaves its fp32 partial tile in `part`; the last of a tile's pieces (completion counter)
-    // adds them in piece order and applies the epilogue.
+    // leaves its fp32 partial tile in `part` and counts itself in.  Of two pieces the last one adds the
+    // other's and applies the epilogue; three or more share the tile's rows out among them.
     int n_full, split;
     // cut > 0 (split 2): a tile's pieces are K steps [0, cut) and [cut, all) (unequal), and the
     // items hold every tile's first piece before any second piece (the long pieces go first; the
@@ -347,12 +347,16 @@ struct PcArgs {
     int cut;
     f32x4* part;                // [(tiles - n_full) * split][32][256] partial tiles
     uint32_t part_bytes;        // their size (the raw buffer's range)
-    uint32_t* counters;         // [tiles - n_full], zero between calls (the last piece resets)
+    // per split tile, cstride words apart: pieces landed; shares claimed, and in the upper half pieces
+    // that gave up waiting.  Zero between calls.
+    uint32_t* counters;
+    int cstride, polls;
     PcGroup g[EXL3_MAX_GROUPS];
 };
 
 struct PC {
     static constexpr int MT = 256, THREADS = 512;
+    static constexpr int POLLS = 48;                   // of a tile's count by a piece's workgroup (~0.7 us each)
     static constexpr int RT_BYTES = 16 * 128;          // one row tile of xh for one K step (2 KB)
     static constexpr int A_BYTES = (MT / 16) * RT_BYTES;   // 32 KB
     static constexpr int B_BYTES = 2 * 8 * FRAG;       // 16 KB
@@ -381,10 +385,10 @@ template <int BITS, int CB>
 __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
 {
     extern __shared__ __align__(16) char lds[];
-    __shared__ int s_last;
+    __shared__ int s_last, s_share;
     const int t = threadIdx.x;
     const int b = blockIdx.x;
-    const bool piece = b >= a.n_full;
+    const bool piece = b >= a.n_full, whole = !piece || a.split == 2;   // whole: one workgroup ends the tile
     int u, q = 0;
     if (!piece) {
         u = a.xcd_remap ? (b & 7) * (a.n_full / 8) + (b >> 3) : b;    // consecutive tiles share an XCD
@@ -418,6 +422,7 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
     // partial tile of piece pq of this tile: consumer thread t's 32 accumulator quads, 16 B apart
     // per thread (coalesced); system-coherent (sc1) accesses, read by another CU after the counter
     const int tile_r = u - a.n_full;
+    uint32_t* const cnt = a.counters + tile_r * a.cstride;     // (pieces only)
     const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(a.part, 0, (int) a.part_bytes, RAW_BUFFER_FLAGS);
     auto part_off = [&](int pq, int ij) __attribute__((always_inline)) {
         return (uint32_t) ((((tile_r * a.split + pq) * 32 + ij) * 256 + t) * 16);
@@ -493,8 +498,7 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
         if (live_rt == 4) main_loop(std::true_type{});
         else main_loop(std::false_type{});
         if (piece) {
-            // this piece's partial out (its live row tiles); then count the pieces in, and the last
-            // one sums them all
+            // this piece's partial out (its live row tiles); then count it in
             if (live_rt == 4) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -515,51 +519,54 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
             __builtin_amdgcn_s_waitcnt(0x0F70);            // vmcnt(0): the partial has landed
             __syncthreads();
             if (t == 0) {
-                const uint32_t prev = __hip_atomic_fetch_add(&a.counters[tile_r], 1u, __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_AGENT);
-                s_last = prev == (uint32_t) (a.split - 1);
-                if (s_last) __hip_atomic_store(&a.counters[tile_r], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                bool all = prev == (uint32_t) (a.split - 1);
+                if (a.split == 2) {
+                    if (all) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } else {
+                    for (int i = 0; i < a.polls && !all; ++i) {
+                        __builtin_amdgcn_s_sleep(2);
+                        all = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t) a.split;
+                    }
+                    s_share = (int) __hip_atomic_fetch_add(cnt + 1, all ? 1u : 0x10000u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                s_last = all;
             }
             __syncthreads();
-            if (!s_last) return;                           // uniform: the whole workgroup leaves
-            // C = sum of the pieces' partials in piece order (this piece's own from registers), 8
-            // accumulator quads at a time: their 8 loads of one piece go out together, one round
-            // trip per piece and batch (a load per quad and piece in turn was 32 x (split - 1)
-            // dependent round trips at the end of the launch)
+            // two pieces: C = the sum, this piece's from registers, 16 quads of the other's in flight
+            // (8 at a time took the gather 3.8 us, 4 round trips)
+            if (a.split == 2 && s_last) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (i >= live_rt) continue;                // dead row tiles: never stored
-                f32x4 sum[8];
-                for (int pq = 0; pq < a.split; ++pq) {
-                    f32x4 v[8];
-                    if (pq == q) {
+                for (int i = 0; i < 4; i += 2) {
+                    if (i >= live_rt) continue;                // dead row tiles: never stored
+                    f32x4 v[2][8];
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) v[j] = acc[i][j];
-                    } else {
+                    for (int h = 0; h < 2; ++h)
 #pragma unroll
                         for (int j = 0; j < 8; ++j)
-                            v[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(prs, part_off(pq, i * 8 + j),
-                                                                                                  0, SC1));
-                    }
+                            v[h][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                prs, i + h < live_rt ? part_off(1 - q, (i + h) * 8 + j) : 0xFFFFFFF0u, 0, SC1));
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) sum[j] = pq == 0 ? v[j] : sum[j] + v[j];
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) acc[i + h][j] += v[h][j];
                 }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc[i][j] = sum[j];
             }
         }
-        // C = fp16(acc) into LDS: every read and write of the stages finished before the last B_s
-        uint16_t* ct = reinterpret_cast<uint16_t*>(lds);
+        if (whole && (!piece || s_last)) {
+            // C = fp16(acc) into LDS: every read and write of the stages finished before the last B_s
+            uint16_t* ct = reinterpret_cast<uint16_t*>(lds);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
+                for (int j = 0; j < 8; ++j)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int r = wave * 64 + i * 16 + 4 * (lane >> 4) + e;
-                    const int c = j * 16 + (lane & 15);
-                    ct[r * PC::C_ROW + c] = f16_bits((f16) acc[i][j][e]);
-                }
+                    for (int e = 0; e < 4; ++e) {
+                        const int r = wave * 64 + i * 16 + 4 * (lane >> 4) + e;
+                        const int c = j * 16 + (lane & 15);
+                        ct[r * PC::C_ROW + c] = f16_bits((f16) acc[i][j][e]);
+                    }
+        }
     } else {
         // ---- producer ---------------------------------------------------------------------
         // the producer is the longer path of a step: its VALU issue goes first (measured faster)
@@ -670,17 +677,22 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
         if (piece) {                                       // the consumers' two completion barriers
             __syncthreads();
             __syncthreads();
-            if (!s_last) return;
         }
     }
-    __syncthreads();                                       // C tile complete in LDS
+
+    if (whole) {
+        if (piece && !s_last) return;                          // uniform: the whole workgroup leaves
+        __syncthreads();                                       // C tile complete in LDS
+    }
 
     // ---- epilogue: y = fp16(fp16(Had128(C)) * svh) on the matrix cores, 16 rows per wave pass
     // (had128_mfma16: the values of exl3_had_r_128_f32 with post), 16-byte stores ----------------
-    const uint16_t* ct = reinterpret_cast<const uint16_t*>(lds);
+    uint16_t* const ctw = reinterpret_cast<uint16_t*>(lds);
+    const uint16_t* const ct = ctw;
     const int jr = t & 15, gq = (t >> 4) & 3;
-    // svh as device-scope (sc1) raw-buffer loads: a split tile's last piece reaches here after its
+    // svh as device-scope (sc1) raw-buffer loads: a split tile's pieces reach here after their
     // counter atomic, and every load after a counter atomic carries sc1 (checked on the built code)
+    // (after the barrier, which would wait for them: 1.5 us a whole tile)
     u32x4 sv[4];
     const __amdgpu_buffer_rsrc_t svs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(gg.svh), 0, 0x7FFFFFFF,
                                                                          RAW_BUFFER_FLAGS);
@@ -693,15 +705,86 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
     const __amdgpu_buffer_rsrc_t ysrc = __builtin_amdgcn_make_buffer_rsrc(gg.y + (int64_t) row0 * a.ldy, 0, 0x7FFFFFFF,
                                                                           RAW_BUFFER_FLAGS);
     const HadMfmaA HA = had_mfma_a();
-    for (int rg = t >> 6; rg < PC::MT / 16 && row0 + 16 * rg < M; rg += PC::THREADS / 64) {
-        const int r = rg * 16 + jr;
-        u32x4 xb[4];
+    auto emit = [&](int rg0, int rg1) __attribute__((always_inline)) {     // 16-row tiles [rg0, rg1) of the tile
+        for (int rg = rg0 + wave; rg < rg1; rg += PC::THREADS / 64) {
+            const int r = rg * 16 + jr;
+            u32x4 xb[4];
 #pragma unroll
-        for (int s_ = 0; s_ < 4; ++s_) xb[s_] = *reinterpret_cast<const u32x4*>(ct + r * PC::C_ROW + 32 * s_ + 8 * gq);
-        had128_mfma16(HA, xb, r_scale<float>(), true, sv, [&](int p, u32x4 v) __attribute__((always_inline)) {
-            if (row0 + r < M)
-                __builtin_amdgcn_raw_buffer_store_b128(v, ysrc, (uint32_t) (((int64_t) r * a.ldy + col0 + 32 * p + 8 * gq) * 2), 0, SC1);
-        });
+            for (int s_ = 0; s_ < 4; ++s_) xb[s_] = *reinterpret_cast<const u32x4*>(ct + r * PC::C_ROW + 32 * s_ + 8 * gq);
+            had128_mfma16(HA, xb, r_scale<float>(), true, sv, [&](int p, u32x4 v) __attribute__((always_inline)) {
+                if (row0 + r < M)
+                    __builtin_amdgcn_raw_buffer_store_b128(v, ysrc, (uint32_t) (((int64_t) r * a.ldy + col0 + 32 * p + 8 * gq) * 2), 0, SC1);
+            });
+        }
+    };
+    const int live = min(PC::MT / 16, (M - row0 + 15) / 16);              // row tiles holding live rows
+    if (whole) {
+        emit(0, live);
+        return;
+    }
+    // ---- a tile of three or more pieces: its rows shared out ------------------------------------
+    // A CU reads the partials at ~65 GB/s however many loads are in flight (20 dependent round trips, or
+    // 128 KB at once, measured the same), so one workgroup summing a whole tile held a launch 10 us
+    // (4 or 6 pieces; 16 us for 10) after its last piece had landed, every other CU idle.  So a piece's
+    // workgroup waits for the others' count, a bounded number of polls (pieces end within a few us
+    // of each other; the last to land waits for nothing), and takes shares of `per` row tiles until none is
+    // left: whoever gave up only leaves more to the rest.  The sums are in piece order whoever takes them.
+    // One summing workgroup / shared out (graphs, transform included, 4 bpw): 5120 -> 1024, 200 rows, 10
+    // pieces 40.2 / 27.0 us; 6144 -> 5120, 200 rows, 6 pieces 40.6 / 33.5; 17408 -> 5120, 200 rows 64.8 / 58.9;
+    // gate/up, 200 rows 114.6 / 102.1; 5120 -> 10240 at 2 bpw, 1024 rows, 4 pieces of the tail 124.7 / 117.3;
+    // 5120 -> 5120, 2048 rows 127.0 / 121.8.  Two pieces are not shared: all CUs reading both partials
+    // back took 59.9 us against 56.5 (5120 -> 5120, 768 rows).
+    const int per = (live + a.split - 1) / a.split, shares = (live + per - 1) / per;
+    int claim = __builtin_amdgcn_readfirstlane(s_share);
+    const bool gave_up = !s_last;
+    while (!gave_up && (claim & 0xFFFF) < shares) {
+        const int rt0 = (claim & 0xFFFF) * per, rt1 = min(live, rt0 + per);
+        // wave w: quad w of every row tile (16 columns); four pieces of four row tiles in flight
+        // (past the last an offset out of the buffer's range: no access, zeros; their rows of the C tile
+        // in LDS, up to RB - 1 row tiles past it, are never read)
+        constexpr int PB = 4, RB = 4;
+        static_assert((PC::MT + 16 * (RB - 1)) * PC::C_ROW * 2 <= PC::LDS, "rows past the tile");
+#pragma unroll 1
+        for (int r0 = rt0; r0 < rt1; r0 += RB) {
+            f32x4 sum[RB];
+#pragma unroll
+            for (int r = 0; r < RB; ++r) sum[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int p0 = 0; p0 < a.split; p0 += PB) {
+                f32x4 v[PB][RB];
+#pragma unroll
+                for (int p = 0; p < PB; ++p)
+#pragma unroll
+                    for (int r = 0; r < RB; ++r) {
+                        const bool has = p0 + p < a.split && r0 + r < rt1;
+                        const uint32_t rt = (uint32_t) (has ? r0 + r : r0), pq = (uint32_t) (has ? p0 + p : p0);
+                        v[p][r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                            prs, has ? (uint32_t) lane * 16u : 0xFFFFFFF0u,
+                            ((((uint32_t) tile_r * a.split + pq) * 32u + (rt & 3u) * 8u + wave) * 256u + (rt >> 2) * 64u) * 16u, SC1));
+                    }
+#pragma unroll
+                for (int p = 0; p < PB; ++p)
+#pragma unroll
+                    for (int r = 0; r < RB; ++r) sum[r] += v[p][r];
+            }
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    ctw[((r0 + r) * 16 + 4 * (lane >> 4) + e) * PC::C_ROW + wave * 16 + (lane & 15)] = f16_bits((f16) sum[r][e]);
+        }
+        __syncthreads();                                       // the share complete in LDS, s_share read
+        emit(rt0, rt1);
+        if (t == 0) s_share = (int) __hip_atomic_fetch_add(cnt + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        claim = __builtin_amdgcn_readfirstlane(s_share);
+    }
+    // every workgroup's last access was a claim that found no share left or its giving up: the one
+    // whose was the last of all clears the counters
+    const int empty = max(0, (claim & 0xFFFF) - shares) + (claim >> 16);   // of the others
+    if (t == 0 && empty == a.split - 1) {
+        __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(cnt + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -724,7 +807,7 @@ int launch_gemm_pc(const PcArgs& a, int items, hipStream_t s)
 // at least 8 K steps (or, below one wave, the two unequal pieces below: at least 5), so the launch
 // ends in balance.  A function of the shape only.
 constexpr int PC_CUS = 256;                    // MI355X compute units
-constexpr size_t PC_COUNTER_BYTES = 4096;      // workspace head: completion counters of split tiles
+constexpr size_t PC_COUNTER_BYTES = 4096;      // workspace head: the split tiles' counters
 constexpr size_t PC_PIECE_BYTES = (size_t) PC::MT * NT_COLS * 4;   // one fp32 partial tile
 
 struct PcPlan {
@@ -804,7 +887,14 @@ int launch_trellis_gemm(const uint16_t* const* xh, int64_t ldx, const void* cons
     a.cut = pl.cut;
     a.xcd_remap = a.n_full % 8 == 0;
     if (pl.split > 1) {
+        // the tiles' counters as far apart as the head has room for (a power of two of words, at most
+        // two 128-byte lines; split tiles: at most 170, 128 of three or more pieces): the polls of
+        // many tiles on one line delayed the other pieces' partials by 4 to 8 us
         a.counters = (uint32_t*) ws;
+        const char* ep = getenv("EXL3_GEMM_POLLS");          // (tests: 0, nobody waits)
+        a.polls = ep ? std::min(std::max(atoi(ep), 0), PC::POLLS) : PC::POLLS;
+        a.cstride = 64;
+        while (a.cstride * (tiles - a.n_full) * 4 > (int) PC_COUNTER_BYTES) a.cstride /= 2;
         a.part = (f32x4*) ((char*) ws + PC_COUNTER_BYTES);
         a.part_bytes = (uint32_t) (pl.ws_bytes - PC_COUNTER_BYTES);
     }

@@ -258,6 +258,8 @@ def check_barriers(insts: list) -> tuple:
                         break
                     if cur.op == "s_waitcnt":
                         thresh = min(thresh, c + _vmcnt(cur.text))
+                        if c >= thresh:                   # c only grows, thresh only falls: all older loads are complete
+                            break
                     elif _VMEM.match(cur.op):
                         if _is_lds_dma(cur):
                             lds += 1
