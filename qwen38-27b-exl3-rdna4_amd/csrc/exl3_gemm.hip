@@ -423,6 +423,10 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
     // per thread (coalesced); system-coherent (sc1) accesses, read by another CU after the counter
     const int tile_r = u - a.n_full;
     uint32_t* const cnt = a.counters + tile_r * a.cstride;     // (pieces only)
+    const int live = min(PC::MT / 16, (M - row0 + 15) / 16);   // 16-row tiles holding live rows
+    // up to 64 live rows of a tile are not worth sharing out: the last workgroup's sums take as long as
+    // the claims (1536 -> 1024, 12 rows: 16.7 us shared, 15.4 not; 100 rows: 19.5 shared, 21.6 not)
+    const bool alone = a.split == 2 || live <= 4;
     const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(a.part, 0, (int) a.part_bytes, RAW_BUFFER_FLAGS);
     auto part_off = [&](int pq, int ij) __attribute__((always_inline)) {
         return (uint32_t) ((((tile_r * a.split + pq) * 32 + ij) * 256 + t) * 16);
@@ -521,7 +525,8 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
             if (t == 0) {
                 const uint32_t prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 bool all = prev == (uint32_t) (a.split - 1);
-                if (a.split == 2) {
+                if (alone) {
+                    s_share = 0;
                     if (all) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 } else {
                     for (int i = 0; i < a.polls && !all; ++i) {
@@ -717,7 +722,6 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
             });
         }
     };
-    const int live = min(PC::MT / 16, (M - row0 + 15) / 16);              // row tiles holding live rows
     if (whole) {
         emit(0, live);
         return;
@@ -734,7 +738,8 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
     // gate/up, 200 rows 114.6 / 102.1; 5120 -> 10240 at 2 bpw, 1024 rows, 4 pieces of the tail 124.7 / 117.3;
     // 5120 -> 5120, 2048 rows 127.0 / 121.8.  Two pieces are not shared: all CUs reading both partials
     // back took 59.9 us against 56.5 (5120 -> 5120, 768 rows).
-    const int per = (live + a.split - 1) / a.split, shares = (live + per - 1) / per;
+    if (alone && !s_last) return;                              // uniform: the whole workgroup leaves
+    const int per = alone ? live : (live + a.split - 1) / a.split, shares = (live + per - 1) / per;
     int claim = __builtin_amdgcn_readfirstlane(s_share);
     const bool gave_up = !s_last;
     while (!gave_up && (claim & 0xFFFF) < shares) {
@@ -775,6 +780,7 @@ __global__ void __launch_bounds__(PC::THREADS) gemm_pc_kernel(PcArgs a)
         }
         __syncthreads();                                       // the share complete in LDS, s_share read
         emit(rt0, rt1);
+        if (alone) return;
         if (t == 0) s_share = (int) __hip_atomic_fetch_add(cnt + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
         claim = __builtin_amdgcn_readfirstlane(s_share);
