@@ -298,8 +298,8 @@ size_t exl3_gemm_trellis_workspace_max(void);
 
 /* Self-check of the register-decode GEMM's unit split for a launch (host only, no GPU): the kernel's
  * 32-bit division forms against brute force.  Returns the number of mismatches (0), or -1 for a shape
- * that GEMM does not serve (more than 128 rows, k below 2048 or not a multiple of 256).  No
- * reference counterpart.  Callers: the CPU tests. */
+ * that GEMM does not serve (more than 128 rows, k below 2048 or not a multiple of 256, m * k from
+ * 2^30 on).  No reference counterpart.  Callers: the CPU tests. */
 int exl3_gemm_rd_check(int m, int k, const int* widths, int groups);
 
 /* Dispatcher by row count: m <= 32 -> fused GEMV, else the prefill GEMM.  Returns the route

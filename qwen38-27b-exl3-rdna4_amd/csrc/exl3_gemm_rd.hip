@@ -566,6 +566,8 @@ RdPlan rd_plan(int M, int K, const int* widths, int groups)
     // K below 2048 stays with the prefill kernel: its launches too short to split are bitwise equal to
     // reconstruct + hgemm and between grouped and single calls, which cut tiles are not
     if (M < 1 || M > RD_MAX_ROWS || K % 256 || K < 2048) return p;
+    // the rotated input of a group is read through a raw buffer with 32-bit byte offsets
+    if ((uint64_t) M * (uint64_t) K * 2 >= (1ull << 31)) return p;
     const int64_t upt = K / 256;
     int64_t tiles = 0;
     for (int i = 0; i < groups; ++i) {

@@ -40,6 +40,15 @@ def test_shapes_not_served():
     assert check(64, 5120, [100]) == -1 and check(64, 5120, [128 * 4097]) == -1 and check(0, 5120, [128]) == -1
 
 
+@pytest.mark.parametrize("m", [33, 64, 128])
+def test_input_range(m):
+    """The rotated input's byte offsets have 32 bits: m * k * 2 stays below 2^31 (the prefill GEMM's 64-bit
+    kernel takes what is larger)."""
+    k = ((1 << 30) - 1) // m // 256 * 256                          # the largest k of that many rows
+    assert check(m, k, [128]) == 0 and check(m, k + 256, [128]) == -1
+    assert check(m, 1 << 25, [128]) == -1
+
+
 def test_workspace_max_holds_every_plan():
     lib = _lib.lib()
     assert lib.exl3_gemm_trellis_workspace_max() == lib.exl3_gemm_trellis_workspace_bound() + 4 * 4096
