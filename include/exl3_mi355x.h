@@ -296,6 +296,11 @@ size_t exl3_gemm_trellis_workspace_bound(void);
  * Callers: exl3rocm's prefill workspace. */
 size_t exl3_gemm_trellis_workspace_max(void);
 
+/* Whether a call of that shape (output rows ldy apart) with exl3_gemm_trellis_workspace_max() bytes of
+ * workspace runs on the register-decode GEMM: 1 or 0 (host only, no GPU).  What it serves at m rows it
+ * serves at fewer.  No reference counterpart.  Callers: exl3rocm's choice between the GEMV and the GEMM. */
+int exl3_gemm_rd_serves(int m, int k, const int* widths, int groups, int K, int64_t ldy);
+
 /* Self-check of the register-decode GEMM's unit split for a launch (host only, no GPU): the kernel's
  * 32-bit division forms against brute force.  Returns the number of mismatches (0), or -1 for a shape
  * that GEMM does not serve (more than 128 rows, k below 2048 or not a multiple of 256, m * k from

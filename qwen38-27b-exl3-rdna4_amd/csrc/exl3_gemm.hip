@@ -917,6 +917,18 @@ int launch_trellis_gemm_cb(int cb, const uint16_t* const* xh, int64_t ldx, const
     return launch_trellis_gemm<BITS, 2>(xh, ldx, tr, y, ldy, svh, widths, groups, M, K, ws, wsb, s);
 }
 
+// Whether the register-decode GEMM serves a call that brings exl3_gemm_trellis_workspace_max() bytes, and
+// its plan: the plan's shapes, partial tiles that fit the workspace, and trellis and output offsets of
+// 32 bits.  Each limit grows with m: what it serves at m rows it serves at fewer.
+bool rd_serves(RdPlan& rd, int m, int k, const int* widths, int groups, int K, int64_t ldy)
+{
+    rd = rd_plan(m, k, widths, groups);
+    bool ok = rd.use && rd.part_bytes <= exl3_gemm_trellis_workspace_bound() - PC_COUNTER_BYTES &&
+              (uint64_t) m * (uint64_t) ldy * 2 < (1ull << 31);
+    for (int i = 0; i < groups; ++i) ok = ok && (uint64_t) k * widths[i] * K / 8 < (1ull << 31);
+    return ok;
+}
+
 // x -> per-group xh (input Hadamards), then one GEMM launch over every group's tiles; x_up (may be
 // null): the input rows are fp16(fp16(silu(x)) * x_up), formed by the transform as it loads them
 int gemm_trellis_common(const void* x, int64_t ldx, const void* const* trellis, uint16_t* const* y, int64_t ldy,
@@ -934,14 +946,11 @@ int gemm_trellis_common(const void* x, int64_t ldx, const void* const* trellis, 
         svs[i] = (const uint16_t*) svh[i];
     }
     const int cb = codebook_of(mcg, mul1);
-    // up to 128 rows the register-decode GEMM (exl3_gemm_rd.hip; its plan says which shapes): its partial
+    // up to 128 rows the register-decode GEMM (exl3_gemm_rd.hip), where it serves the call: its partial
     // tiles in the prefill's, its counters behind them.  EXL3_GEMM_KERNEL set (comparisons): not taken.
     const char* e = getenv("EXL3_GEMM_KERNEL");
     RdPlan rd{};
-    if (ws && wsb >= exl3_gemm_trellis_workspace_max() && !(e && e[0])) rd = rd_plan(m, k, widths, groups);
-    bool use_rd = rd.use && rd.part_bytes <= exl3_gemm_trellis_workspace_bound() - PC_COUNTER_BYTES &&
-                  (uint64_t) m * (uint64_t) ldy * 2 < (1ull << 31);
-    for (int i = 0; i < groups; ++i) use_rd = use_rd && (uint64_t) k * widths[i] * K / 8 < (1ull << 31);
+    const bool use_rd = ws && wsb >= exl3_gemm_trellis_workspace_max() && !(e && e[0]) && rd_serves(rd, m, k, widths, groups, K, ldy);
     // the groups' input transforms (one x, each group's suh) in one launch: the float32 sums of the
     // prefill; the GEMV's exact ones for the register-decode GEMM up to the GEMV's 64 rows
     const int rc = launch_had(x, ldx, xo, k, m, k, suh, groups, nullptr, 1.0f, s, use_rd && m <= EXL3_GEMV_MAX_ROWS, x_up, use_rd);
@@ -1009,6 +1018,15 @@ size_t exl3_gemm_trellis_workspace_bound(void)
 size_t exl3_gemm_trellis_workspace_max(void)
 {
     return exl3_gemm_trellis_workspace_bound() + (size_t) RD_MAX_TILES * sizeof(uint32_t);
+}
+
+int exl3_gemm_rd_serves(int m, int k, const int* widths, int groups, int K, int64_t ldy)
+{
+    if (!widths || groups < 1 || groups > EXL3_MAX_GROUPS || K < 1 || K > 8 || ldy < 0) return 0;
+    for (int i = 0; i < groups; ++i)
+        if (widths[i] < 128 || widths[i] % 128) return 0;
+    RdPlan rd{};
+    return rd_serves(rd, m, k, widths, groups, K, ldy);
 }
 
 int exl3_gemm_trellis_grouped(const void* x, int64_t ldx, const void* const* trellis, void* y, int64_t ldy,

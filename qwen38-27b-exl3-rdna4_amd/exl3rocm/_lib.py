@@ -56,6 +56,7 @@ SIGNATURES = {
     "exl3_gemm_trellis_workspace_size": (_sz, [_i, _i, _ip, _i]),
     "exl3_gemm_trellis_workspace_bound": (_sz, []),
     "exl3_gemm_trellis_workspace_max": (_sz, []),
+    "exl3_gemm_rd_serves": (_i, [_i, _i, _ip, _i, _i, _i64]),
     "exl3_gemm_rd_check": (_i, [_i, _i, C.POINTER(C.c_int), _i]),
     "exl3_gemm": (_i, [_p, _i64, _p, _p, _i64, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _sz, _p]),
     "exl3_gemv_mr_approx": (_i, [_p, _i64, _p, _p, _i64, _p, _p, _p, _i, _i, _i, _i, _i, _p, _sz, _p]),

@@ -19,7 +19,9 @@ or EXL3_MR_MAX rows for every shape when set):
 """
 from __future__ import annotations
 
+import functools
 import os
+from ctypes import c_int as C_int
 from typing import Optional
 
 import torch
@@ -33,13 +35,15 @@ def _env_rows(name: str) -> Optional[int]:
 
 
 # EXL3_MR_MAX (the reference's knob) fixes the GEMV / GEMM boundary for every launch; unset, each launch
-# takes the measured crossover of its shape from GEMV_CROSSOVER, or for shapes outside it MID_MR where
-# the register-decode GEMM takes over (k a multiple of 256 from MID_K), else DEFAULT_MR
+# takes a measured crossover of its shape: against the register-decode GEMM (up to 128 rows) where that
+# serves the launch, else against the prefill GEMM
 MR_MAX: Optional[int] = _env_rows("EXL3_MR_MAX")
+# the library's comparison knob; set, the register-decode GEMM is not taken
+GEMM_KERNEL = os.environ.get("EXL3_GEMM_KERNEL", "")
 DEFAULT_MR = 32
 MID_MR, MID_K = 8, 3072
-# Largest row count at which the fused GEMV beats the GEMM route, by (k, output columns of the launch:
-# all its groups).  Measured on MI355X for the launches a Qwen3.5-27B checkpoint makes (q/k/v and
+# Largest row count at which the fused GEMV beats the register-decode GEMM, by (k, output columns of the
+# launch: all its groups).  Measured on MI355X for the launches a Qwen3.5-27B checkpoint makes (q/k/v and
 # gate/up grouped as linear_groups groups them, and lm_head) and 4096 x 4096: both routes at 20 row
 # counts from 2 to 64, graphs of 16 launches over cold weights, 4 bpw, and 2 / 3 / 5 bpw where a
 # checkpoint holds them.  The GEMV's cost grows with every row, the register-decode GEMM's (up to
@@ -56,25 +60,51 @@ GEMV_CROSSOVER = {
     (5120, 10240): 8, (5120, 12288): 8, (5120, 14336): 8, (5120, 16384): 8, (5120, 17408): 8,
     (5120, 34816): 8, (5120, 248320): 32, (6144, 5120): 8, (17408, 5120): 8,
 }
+# The same against the prefill GEMM (other shapes: DEFAULT_MR), for launches that the register-decode GEMM
+# does not serve: both routes at every row count from 2 to 64, graphs of 24 launches over 8 weight
+# copies, 4 bpw, and 2 / 3 bpw where a checkpoint holds them (the boundary moved by <= 4 rows).  Each
+# entry is within 1 % of the least summed time, with no step above 5 % from the GEMV to the GEMM: the
+# prefill GEMM's cost is flat within each 16-row MFMA tile, so it wins early where its 128-column tiles fill
+# the chip (5120 - 7168 columns: 17 - 19) and late where they do not (the k/v launches, 2 x 17408 columns
+# and lm_head: 58 to the GEMV's 64-row limit).
+PREFILL_CROSSOVER = {
+    (5120, 1024): 64, (5120, 2048): 58, (5120, 5120): 17, (5120, 6144): 17, (5120, 7168): 19,
+    (5120, 10240): 31, (5120, 12288): 33, (5120, 14336): 25, (5120, 16384): 33, (5120, 17408): 46,
+    (5120, 34816): 64, (5120, 248320): 64, (6144, 5120): 30, (17408, 5120): 39,
+}
 
 
-def gemv_max_rows(k: int, width: int) -> int:
-    """Most rows a launch of k inputs and `width` output columns takes on the fused GEMV."""
+@functools.lru_cache(maxsize=4096)
+def _rd_serves(k: int, widths: tuple, K: int, ldy: int) -> bool:
+    """Whether the library's register-decode GEMM serves such a launch at every row count of the GEMV."""
+    return bool(_lib.lib().exl3_gemm_rd_serves(_lib.GEMV_MAX_ROWS, k, (C_int * len(widths))(*widths), len(widths), K, ldy))
+
+
+def gemv_max_rows(k: int, width: int, K: int = 4, widths: Optional[tuple] = None, ldy: Optional[int] = None) -> int:
+    """Most rows a launch of k inputs and `width` output columns (groups of `widths`, output rows ldy
+    apart) takes on the fused GEMV.  Where the register-decode GEMM is not what the other route runs
+    (EXL3_PREFILL=recon, EXL3_GEMM_KERNEL, shapes beyond its limits) the boundary is the prefill
+    GEMM's: the register-decode GEMM's own is up to 56 rows lower."""
     if MR_MAX is not None:
         return MR_MAX
-    dflt = MID_MR if k >= MID_K and k % 256 == 0 else DEFAULT_MR
-    return min(GEMV_CROSSOVER.get((k, width), dflt), _lib.GEMV_MAX_ROWS)
+    if PREFILL_ROUTE == "recon" or GEMM_KERNEL or not _rd_serves(k, widths or (width,), K, ldy or width):
+        b = PREFILL_CROSSOVER.get((k, width), DEFAULT_MR)
+    else:
+        b = GEMV_CROSSOVER.get((k, width), MID_MR if k >= MID_K and k % 256 == 0 else DEFAULT_MR)
+    return min(b, _lib.GEMV_MAX_ROWS)
 
 
-def gemv_rows(m: int, k: int, width: int) -> bool:
+def gemv_rows(m: int, k: int, width: int, K: int = 4, widths: Optional[tuple] = None, ldy: Optional[int] = None) -> bool:
     """Route of an m-row launch: the fused GEMV (True; every row bitwise equal to its m = 1 call)
-    or the prefill GEMM."""
-    return m <= gemv_max_rows(k, width)
+    or a GEMM."""
+    if MR_MAX is None and m <= MID_MR:                        # no boundary is lower
+        return True
+    return m <= gemv_max_rows(k, width, K, widths, ldy)
 
 
-def fused_rows(m: int, k: int, width: int) -> bool:
+def fused_rows(m: int, k: int, width: int, K: int = 4, widths: Optional[tuple] = None, ldy: Optional[int] = None) -> bool:
     """The GEMV route for the fused-epilogue forms (SiLU input, gated, approximate): <= 32 rows."""
-    return m <= min(gemv_max_rows(k, width), _lib.GEMV_FUSED_MAX_ROWS)
+    return m <= _lib.GEMV_FUSED_MAX_ROWS and gemv_rows(m, k, width, K, widths, ldy)
 
 
 # widest non-lm_head layer (17408): the shared reconstruction buffer of the `recon` prefill route
@@ -123,12 +153,13 @@ def _weight_buffer(device, numel):
 
 
 def reserve_workspace(device, k: int, n: int, K: int, groups: int = 1, m: Optional[int] = None):
-    """Reserve the GEMV workspace for up to m rows (load time; default: the most rows gemv_rows
+    """Reserve the GEMV workspace for up to m rows (load time; default: the most rows that any route
     sends to the GEMV for a module of groups x n columns): the current stream gets it now, and
     every other stream gets at least this much on its first eager call (so a later graph capture on
     that stream never allocates)."""
     if m is None:
-        m = gemv_max_rows(k, n * groups)
+        m = MR_MAX if MR_MAX is not None else max(PREFILL_CROSSOVER.get((k, n * groups), DEFAULT_MR),
+                                                  gemv_max_rows(k, n * groups, K))
     if m < 1:
         return
     E.workspace(torch.device(device), E.gemv_workspace_bytes(min(m, _lib.GEMV_MAX_ROWS), k, n, K, groups),
@@ -151,7 +182,7 @@ def _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y, gemv: Optional[bool] = 
     M, k = x2.shape
     n = svh.shape[0]
     if gemv is None:
-        gemv = gemv_rows(M, k, n)
+        gemv = gemv_rows(M, k, n, K, (n,), y.stride(0))
     if gemv and GEMV_APPROX and mul1 and M <= _lib.GEMV_FUSED_MAX_ROWS:
         rc = E.exl3_gemv_mr_approx(x2, trellis, y, suh, None, svh, K, GEMV_APPROX)
         if rc != 0:
@@ -235,7 +266,7 @@ def _linear_groups(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch
         while j < ng and j - i < _lib.MAX_GROUPS and K[j] == K[i]:
             j += 1
         w = sum(widths[i:j])
-        gemv = gemv_rows(M, k, w)
+        gemv = gemv_rows(M, k, w, K[i], tuple(widths[i:j]), y.stride(0))
         if j == i + 1 or (gemv and GEMV_APPROX and mul1 and M <= _lib.GEMV_FUSED_MAX_ROWS) or \
                 (not gemv and PREFILL_ROUTE == "recon"):
             # one group, the approximate GEMV or the recon prefill: each group its own launch
@@ -291,7 +322,7 @@ def exl3_linear_silu_mul(x: torch.Tensor, trellis: list[torch.Tensor], suh: list
     act = torch.empty((M, n), dtype=torch.float16, device=x.device)
     if M == 0:
         return act.view(*x.shape[:-1], n)
-    if GATED_ROUTE == "fused" and K[0] == K[1] and fused_rows(M, k, 2 * n):
+    if GATED_ROUTE == "fused" and K[0] == K[1] and fused_rows(M, k, 2 * n, K[0], (n, n)):
         E.exl3_gemv_silu_mul(x2, list(trellis), act, list(suh), list(svh), K[0], mcg, mul1)
     else:
         gu = _linear_groups(x2, trellis, suh, svh, K, mcg, mul1)
@@ -327,11 +358,11 @@ def exl3_silu_mul_linear(gu: torch.Tensor, trellis: torch.Tensor, suh: torch.Ten
     y = torch.empty((M, n), dtype=torch.float16, device=gu.device)
     if M == 0:
         return y.view(*gu.shape[:-1], n)
-    if fused_rows(M, k, n) and not (GEMV_APPROX and mul1):
+    if fused_rows(M, k, n, K) and not (GEMV_APPROX and mul1):
         rc = E.exl3_gemv_silu_in(g2[:, :k], g2[:, k:], trellis, y, suh, None, svh, K, mcg, mul1)
         if rc != 0:
             raise RuntimeError(f"exl3rocm: GEMV declined shape m={M} k={k} n={n} K={K}")
-    elif not gemv_rows(M, k, n) and PREFILL_ROUTE != "recon":
+    elif not gemv_rows(M, k, n, K) and PREFILL_ROUTE != "recon":
         xh = torch.empty((M, k), dtype=torch.float16, device=gu.device)
         E.exl3_gemm_trellis_silu_in(g2[:, :k], g2[:, k:], trellis, y, suh, xh, svh, K, mcg, mul1)
     else:

@@ -1,0 +1,82 @@
+"""The route of a launch (GEMV, register-decode GEMM, prefill GEMM), on the CPU: the GEMV keeps its boundary
+against the prefill GEMM wherever the register-decode GEMM is not what the other route runs."""
+import ctypes
+
+import pytest
+import torch
+
+from exl3rocm import _lib, ops
+from test_host import _Launches
+
+CHECKPOINT = sorted(ops.GEMV_CROSSOVER)
+
+
+def serves(m, k, widths, K, ldy=None):
+    return _lib.lib().exl3_gemm_rd_serves(m, k, (ctypes.c_int * len(widths))(*widths), len(widths), K, ldy or sum(widths))
+
+
+@pytest.fixture(autouse=True)
+def defaults(monkeypatch):
+    for name, value in (("MR_MAX", None), ("PREFILL_ROUTE", "fused"), ("GEMM_KERNEL", ""), ("GEMV_APPROX", ""), ("GATED_ROUTE", "unfused")):
+        monkeypatch.setattr(ops, name, value)
+
+
+def test_boundaries():
+    """No boundary below MID_MR (gemv_rows answers those rows at once), none against the prefill GEMM
+    below the one against the register-decode GEMM, which starts to win earlier."""
+    assert sorted(ops.PREFILL_CROSSOVER) == CHECKPOINT
+    for s in CHECKPOINT:
+        assert ops.MID_MR <= ops.GEMV_CROSSOVER[s] <= ops.PREFILL_CROSSOVER[s] <= _lib.GEMV_MAX_ROWS
+    assert ops.MID_MR <= ops.DEFAULT_MR
+
+
+@pytest.mark.parametrize("knob,value", [("PREFILL_ROUTE", "recon"), ("GEMM_KERNEL", "tile"), ("GEMM_KERNEL", "pc")])
+def test_knobs_that_take_another_gemm(monkeypatch, knob, value):
+    """EXL3_PREFILL=recon rebuilds the whole weight on each call and EXL3_GEMM_KERNEL takes the prefill's
+    kernels: the GEMV's rows end where those begin to win."""
+    monkeypatch.setattr(ops, knob, value)
+    for (k, w), b in ops.PREFILL_CROSSOVER.items():
+        assert ops.gemv_rows(b, k, w) and not ops.gemv_rows(b + 1, k, w), (k, w)
+    assert ops.gemv_rows(32, 4096, 4096) and not ops.gemv_rows(33, 4096, 4096)
+    assert ops.fused_rows(30, 6144, 5120) and not ops.fused_rows(31, 6144, 5120) and not ops.fused_rows(33, 17408, 5120)
+
+
+@pytest.mark.parametrize("k,widths,K,ldy", [(8192, (262144,), 8, None),         # a trellis of 2 GiB
+                                            (8192, (262144, 128), 8, None),
+                                            (5120, (128 * 4097,), 1, None),     # more tiles than counters
+                                            (4096, (4096,), 4, 1 << 24),        # output rows too far apart
+                                            (1 << 24, (128,), 1, None)])        # 64 rows of input: 2 GiB
+def test_launches_beyond_the_register_decode_gemm(k, widths, K, ldy):
+    w = sum(widths)
+    assert not serves(64, k, widths, K, ldy)
+    for m in (9, 16, 32):
+        assert ops.gemv_rows(m, k, w, K, widths, ldy), m
+    assert not ops.gemv_rows(33, k, w, K, widths, ldy)
+
+
+def test_serves_fewer_rows_too():
+    """The boundary asks at the GEMV's most rows: what is served there is served at fewer."""
+    for k, widths, K in ((5120, (5120,), 4), (5120, (248320,), 4), (3072, (128,), 1), (17408, (128 * 300, 128), 8), (2048, (128 * 4096,), 2)):
+        assert serves(64, k, widths, K)
+        assert all(serves(m, k, widths, K) for m in range(1, 64))
+    assert not serves(0, 5120, (5120,), 4) and not serves(129, 5120, (5120,), 4) and not serves(64, 5120, (5120,), 9)
+    assert not serves(64, 5120, (100,), 4)
+
+
+def launches(monkeypatch, widths, Ks, m, k=5120):
+    rec = _Launches()
+    monkeypatch.setattr(ops, "E", rec)
+    monkeypatch.setattr(ops, "_weight_buffer", lambda dev, n: torch.empty(n, dtype=torch.float16))
+    tr = [torch.zeros(k // 16, n // 16, 16 * K, dtype=torch.int16) for n, K in zip(widths, Ks)]
+    su = [torch.ones(k, dtype=torch.float16)] * len(widths)
+    sv = [torch.ones(n, dtype=torch.float16) for n in widths]
+    y = torch.ops.exl3rocm.linear_groups(torch.zeros(m, k, dtype=torch.float16), tr, su, sv, list(Ks), False, True)
+    assert tuple(y.shape) == (m, sum(widths))
+    return [name for name, _ in rec.calls]
+
+
+def test_groups_under_recon(monkeypatch):
+    monkeypatch.setattr(ops, "PREFILL_ROUTE", "recon")
+    assert launches(monkeypatch, (1024, 1024), (5, 5), 40) == ["exl3_gemv_mr_grouped"]
+    monkeypatch.setattr(ops, "PREFILL_ROUTE", "fused")
+    assert launches(monkeypatch, (1024, 1024), (5, 5), 40) == ["exl3_gemm_trellis_grouped"]
