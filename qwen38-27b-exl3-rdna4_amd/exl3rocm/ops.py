@@ -80,31 +80,35 @@ def _rd_serves(k: int, widths: tuple, K: int, ldy: int) -> bool:
     return bool(_lib.lib().exl3_gemm_rd_serves(_lib.GEMV_MAX_ROWS, k, (C_int * len(widths))(*widths), len(widths), K, ldy))
 
 
-def gemv_max_rows(k: int, width: int, K: int = 4, widths: Optional[tuple] = None, ldy: Optional[int] = None) -> int:
+def gemv_max_rows(k: int, width: int, K: int = 4, widths: Optional[tuple] = None, ldy: Optional[int] = None,
+                  hold: bool = False) -> int:
     """Most rows a launch of k inputs and `width` output columns (groups of `widths`, output rows ldy
     apart) takes on the fused GEMV.  Where the register-decode GEMM is not what the other route runs
     (EXL3_PREFILL=recon, EXL3_GEMM_KERNEL, shapes beyond its limits) the boundary is the prefill
-    GEMM's: the register-decode GEMM's own is up to 56 rows lower."""
+    GEMM's: the register-decode GEMM's own is up to 56 rows lower.  hold: that boundary for a form of the
+    GEMV that the user asked for by a knob (the approximate and the gated one)."""
     if MR_MAX is not None:
         return MR_MAX
-    if PREFILL_ROUTE == "recon" or GEMM_KERNEL or not _rd_serves(k, widths or (width,), K, ldy or width):
+    if hold or PREFILL_ROUTE == "recon" or GEMM_KERNEL or not _rd_serves(k, widths or (width,), K, ldy or width):
         b = PREFILL_CROSSOVER.get((k, width), DEFAULT_MR)
     else:
         b = GEMV_CROSSOVER.get((k, width), MID_MR if k >= MID_K and k % 256 == 0 else DEFAULT_MR)
     return min(b, _lib.GEMV_MAX_ROWS)
 
 
-def gemv_rows(m: int, k: int, width: int, K: int = 4, widths: Optional[tuple] = None, ldy: Optional[int] = None) -> bool:
+def gemv_rows(m: int, k: int, width: int, K: int = 4, widths: Optional[tuple] = None, ldy: Optional[int] = None,
+              hold: bool = False) -> bool:
     """Route of an m-row launch: the fused GEMV (True; every row bitwise equal to its m = 1 call)
     or a GEMM."""
     if MR_MAX is None and m <= MID_MR:                        # no boundary is lower
         return True
-    return m <= gemv_max_rows(k, width, K, widths, ldy)
+    return m <= gemv_max_rows(k, width, K, widths, ldy, hold)
 
 
-def fused_rows(m: int, k: int, width: int, K: int = 4, widths: Optional[tuple] = None, ldy: Optional[int] = None) -> bool:
+def fused_rows(m: int, k: int, width: int, K: int = 4, widths: Optional[tuple] = None, ldy: Optional[int] = None,
+               hold: bool = False) -> bool:
     """The GEMV route for the fused-epilogue forms (SiLU input, gated, approximate): <= 32 rows."""
-    return m <= _lib.GEMV_FUSED_MAX_ROWS and gemv_rows(m, k, width, K, widths, ldy)
+    return m <= _lib.GEMV_FUSED_MAX_ROWS and gemv_rows(m, k, width, K, widths, ldy, hold)
 
 
 # widest non-lm_head layer (17408): the shared reconstruction buffer of the `recon` prefill route
@@ -127,8 +131,13 @@ def approx_mode(value: Optional[str]) -> str:
     return v
 
 
-# opt-in approximate mul1 GEMV, in place of the faithful one where fused_rows holds
+# opt-in approximate mul1 GEMV, up to 32 rows of the boundary against the prefill GEMM (fused_rows, hold)
 GEMV_APPROX = approx_mode(os.environ.get("EXL3_GEMV_APPROX"))
+
+
+def _approx(m: int, mul1: bool) -> bool:
+    return bool(GEMV_APPROX) and mul1 and m <= _lib.GEMV_FUSED_MAX_ROWS
+
 
 _wbuf: dict = {}
 
@@ -182,8 +191,8 @@ def _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y, gemv: Optional[bool] = 
     M, k = x2.shape
     n = svh.shape[0]
     if gemv is None:
-        gemv = gemv_rows(M, k, n, K, (n,), y.stride(0))
-    if gemv and GEMV_APPROX and mul1 and M <= _lib.GEMV_FUSED_MAX_ROWS:
+        gemv = gemv_rows(M, k, n, K, (n,), y.stride(0), _approx(M, mul1))
+    if gemv and _approx(M, mul1):
         rc = E.exl3_gemv_mr_approx(x2, trellis, y, suh, None, svh, K, GEMV_APPROX)
         if rc != 0:
             raise RuntimeError(f"exl3rocm: approximate GEMV declined shape m={M} k={k} n={n} K={K}")
@@ -259,15 +268,18 @@ def _linear_groups(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch
         return x2.new_empty((*x.shape[:-1], sum(widths)), dtype=torch.float16)
     y = torch.empty((M, sum(widths)), dtype=torch.float16, device=x.device)
     # runs of consecutive groups with equal K share one launch, each group written straight into
-    # its row-strided column slice; each run takes the route of its own shape
+    # its row-strided column slice; each run takes the route of its own shape (EXL3_GATED=fused: gate and
+    # up that of their one-launch form, so that both stay bitwise the same)
+    hold = _approx(M, mul1) or (GATED_ROUTE == "fused" and ng == 2 and K[0] == K[1] and widths[0] == widths[1]
+                                and M <= _lib.GEMV_FUSED_MAX_ROWS)
     i, n0 = 0, 0
     while i < ng:
         j = i + 1
         while j < ng and j - i < _lib.MAX_GROUPS and K[j] == K[i]:
             j += 1
         w = sum(widths[i:j])
-        gemv = gemv_rows(M, k, w, K[i], tuple(widths[i:j]), y.stride(0))
-        if j == i + 1 or (gemv and GEMV_APPROX and mul1 and M <= _lib.GEMV_FUSED_MAX_ROWS) or \
+        gemv = gemv_rows(M, k, w, K[i], tuple(widths[i:j]), y.stride(0), hold)
+        if j == i + 1 or (gemv and _approx(M, mul1)) or \
                 (not gemv and PREFILL_ROUTE == "recon"):
             # one group, the approximate GEMV or the recon prefill: each group its own launch
             c = n0
@@ -322,7 +334,7 @@ def exl3_linear_silu_mul(x: torch.Tensor, trellis: list[torch.Tensor], suh: list
     act = torch.empty((M, n), dtype=torch.float16, device=x.device)
     if M == 0:
         return act.view(*x.shape[:-1], n)
-    if GATED_ROUTE == "fused" and K[0] == K[1] and fused_rows(M, k, 2 * n, K[0], (n, n)):
+    if GATED_ROUTE == "fused" and K[0] == K[1] and fused_rows(M, k, 2 * n, K[0], (n, n), hold=True):
         E.exl3_gemv_silu_mul(x2, list(trellis), act, list(suh), list(svh), K[0], mcg, mul1)
     else:
         gu = _linear_groups(x2, trellis, suh, svh, K, mcg, mul1)
@@ -358,17 +370,19 @@ def exl3_silu_mul_linear(gu: torch.Tensor, trellis: torch.Tensor, suh: torch.Ten
     y = torch.empty((M, n), dtype=torch.float16, device=gu.device)
     if M == 0:
         return y.view(*gu.shape[:-1], n)
-    if fused_rows(M, k, n, K) and not (GEMV_APPROX and mul1):
+    approx = _approx(M, mul1)
+    gemv = gemv_rows(M, k, n, K, hold=approx)
+    if gemv and M <= _lib.GEMV_FUSED_MAX_ROWS and not approx:
         rc = E.exl3_gemv_silu_in(g2[:, :k], g2[:, k:], trellis, y, suh, None, svh, K, mcg, mul1)
         if rc != 0:
             raise RuntimeError(f"exl3rocm: GEMV declined shape m={M} k={k} n={n} K={K}")
-    elif not gemv_rows(M, k, n, K) and PREFILL_ROUTE != "recon":
+    elif not gemv and PREFILL_ROUTE != "recon":
         xh = torch.empty((M, k), dtype=torch.float16, device=gu.device)
         E.exl3_gemm_trellis_silu_in(g2[:, :k], g2[:, k:], trellis, y, suh, xh, svh, K, mcg, mul1)
     else:
         act = torch.empty((M, k), dtype=torch.float16, device=gu.device)
         E.silu_mul(g2[:, :k], g2[:, k:], act)
-        _linear_into(act, trellis, suh, svh, K, mcg, mul1, y)
+        _linear_into(act, trellis, suh, svh, K, mcg, mul1, y, gemv)
     return y.view(*gu.shape[:-1], n)
 
 

@@ -80,3 +80,69 @@ def test_groups_under_recon(monkeypatch):
     assert launches(monkeypatch, (1024, 1024), (5, 5), 40) == ["exl3_gemv_mr_grouped"]
     monkeypatch.setattr(ops, "PREFILL_ROUTE", "fused")
     assert launches(monkeypatch, (1024, 1024), (5, 5), 40) == ["exl3_gemm_trellis_grouped"]
+
+
+@pytest.mark.parametrize("m,k,n,approx", [(9, 5120, 17408, True), (32, 5120, 17408, True), (33, 5120, 17408, False),
+                                          (17, 5120, 5120, True), (18, 5120, 5120, False), (32, 4096, 4096, True)])
+def test_approximate_gemv_keeps_its_rows(monkeypatch, m, k, n, approx):
+    """EXL3_GEMV_APPROX: up to 32 rows of the boundary against the prefill GEMM, in every op; mcg and
+    3inst modules take the faithful routes."""
+    monkeypatch.setattr(ops, "GEMV_APPROX", "affine")
+    want = "exl3_gemv_mr_approx" if approx else "exl3_gemm_trellis_grouped"
+    assert launches(monkeypatch, (n,), (4,), m, k) == [want]
+    rec = _Launches()
+    monkeypatch.setattr(ops, "E", rec)
+    t, su, sv = torch.zeros(k // 16, n // 16, 64, dtype=torch.int16), torch.ones(k, dtype=torch.float16), torch.ones(n, dtype=torch.float16)
+    x = torch.zeros(m, k, dtype=torch.float16)
+    torch.ops.exl3rocm.linear(x, t, su, sv, 4, True, False)
+    assert rec.calls.pop()[0] == "exl3_gemm_trellis_grouped"
+    torch.ops.exl3rocm.linear(x, t, su, sv, 4, False, True)
+    assert rec.calls.pop()[0] == want
+
+
+class _Mlp(_Launches):
+    """_Launches for the SiLU forms too, whose arguments lie elsewhere."""
+
+    def __getattr__(self, name):
+        def launch(*args, **kw):
+            self.calls.append((name, None))
+            return 0
+        return launch
+
+
+@pytest.mark.parametrize("m", [9, 30, 31, 32, 33, 40])
+def test_silu_input_forms(monkeypatch, m):
+    """The down projection: the approximate GEMV forms up to their rows, else the GEMM's SiLU input."""
+    k, n = 6144, 5120                                             # boundary against the prefill GEMM: 30
+    gu, t = torch.zeros(m, 2 * k, dtype=torch.float16), torch.zeros(k // 16, n // 16, 64, dtype=torch.int16)
+    su, sv = torch.ones(k, dtype=torch.float16), torch.ones(n, dtype=torch.float16)
+    rec = _Mlp()
+    monkeypatch.setattr(ops, "E", rec)
+    torch.ops.exl3rocm.silu_mul_linear(gu, t, su, sv, 4, False, True)
+    assert [c for c, _ in rec.calls] == ["exl3_gemm_trellis_silu_in"]
+    monkeypatch.setattr(ops, "GEMV_APPROX", "affine")
+    rec.calls.clear()
+    torch.ops.exl3rocm.silu_mul_linear(gu, t, su, sv, 4, False, True)
+    assert [c for c, _ in rec.calls] == (["silu_mul", "exl3_gemv_mr_approx"] if m <= 30 else ["exl3_gemm_trellis_silu_in"])
+
+
+@pytest.mark.parametrize("m", [8, 9, 32, 33])
+def test_gated_form_keeps_its_rows(monkeypatch, m):
+    """EXL3_GATED=fused: the one-launch form up to 32 rows, and linear_groups of gate and up on the GEMV at
+    those rows, whose bits it has; without the knob both take the GEMM from 9 rows."""
+    k, n = 5120, 17408
+    x, t = torch.zeros(m, k, dtype=torch.float16), torch.zeros(k // 16, n // 16, 64, dtype=torch.int16)
+    su, sv = torch.ones(k, dtype=torch.float16), torch.ones(n, dtype=torch.float16)
+
+    def calls(op):
+        rec = _Mlp()
+        monkeypatch.setattr(ops, "E", rec)
+        op(x, [t, t], [su, su], [sv, sv], [4, 4], False, True)
+        return [c for c, _ in rec.calls]
+
+    small = "exl3_gemv_mr_grouped" if m <= 8 else "exl3_gemm_trellis_grouped"
+    assert calls(torch.ops.exl3rocm.linear_groups) == [small] and calls(torch.ops.exl3rocm.linear_silu_mul) == [small, "silu_mul"]
+    monkeypatch.setattr(ops, "GATED_ROUTE", "fused")
+    fused = m <= 32
+    assert calls(torch.ops.exl3rocm.linear_groups) == (["exl3_gemv_mr_grouped"] if fused else ["exl3_gemm_trellis_grouped"])
+    assert calls(torch.ops.exl3rocm.linear_silu_mul) == (["exl3_gemv_silu_mul"] if fused else ["exl3_gemm_trellis_grouped", "silu_mul"])
