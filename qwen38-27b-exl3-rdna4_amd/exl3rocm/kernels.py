@@ -54,7 +54,9 @@ def workspace(device: torch.device, nbytes: int, stream: Optional[int] = None, r
     which also raises the device's reserved size.  A stream's first eager call then allocates
     that whole reserved size, not just its own call's, so the serving sequence (load, eager
     warm-up on stream S, graph capture on S) never needs an allocation during capture, on any
-    stream.  During capture a stream without a large enough workspace raises."""
+    stream.  Where a layer has reserved the prefill workspace too, the stream gets its own of that with
+    the same call, whatever its rows: a capture there at more rows than were warmed up runs what an
+    eager call runs.  During capture a stream without a large enough workspace raises."""
     if not isinstance(device, torch.device):
         device = torch.device(device)
     if stream is None:
@@ -68,10 +70,13 @@ def workspace(device: torch.device, nbytes: int, stream: Optional[int] = None, r
               "GEMV workspace: this stream made no eager call of this size before graph capture")
         buf = torch.zeros(max(nbytes, _reserved.get(device, 0), 4096), dtype=torch.uint8, device=device)
         _workspaces[key] = buf
+        if device in _pf_reserved:
+            prefill_workspace(device, prefill_workspace_bound(), stream)
     return buf
 
 
 _pf_workspaces: dict = {}
+_pf_reserved: set = set()   # devices on which a layer reserved the prefill workspace
 _pf_bound = None
 
 
@@ -87,9 +92,10 @@ def prefill_workspace(device: torch.device, nbytes: int, stream: Optional[int] =
     """Zeroed workspace of the prefill GEMM's split tail and the register-decode GEMM's partial tiles
     for the current (or given) stream.  A stream's first call outside graph capture allocates the
     size every shape fits in (exl3_gemm_trellis_workspace_max), so a later capture on that stream
-    splits exactly as eager calls do.  A stream that captures before any eager prefill call has
-    none: its launches run unsplit, and the split tiles' outputs can differ from the eager ones' in
-    the last place (another fp32 summation order)."""
+    splits exactly as eager calls do.  A stream that captures without one gets None: the ops keep up to
+    64 rows on the GEMV there as far as it beats the prefill GEMM (ops.gemv_max_rows), and more rows run the
+    prefill GEMM unsplit, with its float32 transforms also at 33 to 64 rows, where eager calls run the
+    register-decode GEMM's exact ones: equal to the tolerance, not bitwise."""
     if nbytes <= 0:
         return None
     if not isinstance(device, torch.device):
@@ -107,8 +113,15 @@ def prefill_workspace(device: torch.device, nbytes: int, stream: Optional[int] =
 
 
 def reserve_prefill_workspace(device: torch.device, stream: Optional[int] = None) -> None:
-    """Allocate the current (or given) stream's prefill workspace now (load time)."""
+    """Allocate the current (or given) stream's prefill workspace now (load time), and every other
+    stream's of the device with its GEMV workspace, on its first eager call."""
+    _pf_reserved.add(torch.device(device))
     prefill_workspace(device, prefill_workspace_bound(), stream)
+
+
+def captures_without_prefill_workspace(x: torch.Tensor) -> bool:
+    """Whether the current stream captures a graph and has no prefill workspace."""
+    return x.is_cuda and torch.cuda.is_current_stream_capturing() and (x.device, _stream(x)) not in _pf_workspaces
 
 
 def gemv_workspace_bytes(m: int, k: int, n: int, K: int, groups: int = 1) -> int:

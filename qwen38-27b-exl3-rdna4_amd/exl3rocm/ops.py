@@ -85,8 +85,7 @@ def gemv_max_rows(k: int, width: int, K: int = 4, widths: Optional[tuple] = None
     """Most rows a launch of k inputs and `width` output columns (groups of `widths`, output rows ldy
     apart) takes on the fused GEMV.  Where the register-decode GEMM is not what the other route runs
     (EXL3_PREFILL=recon, EXL3_GEMM_KERNEL, shapes beyond its limits) the boundary is the prefill
-    GEMM's: the register-decode GEMM's own is up to 56 rows lower.  hold: that boundary for a form of the
-    GEMV that the user asked for by a knob (the approximate and the gated one)."""
+    GEMM's: the register-decode GEMM's own is up to 56 rows lower.  hold: that boundary (_hold)."""
     if MR_MAX is not None:
         return MR_MAX
     if hold or PREFILL_ROUTE == "recon" or GEMM_KERNEL or not _rd_serves(k, widths or (width,), K, ldy or width):
@@ -137,6 +136,17 @@ GEMV_APPROX = approx_mode(os.environ.get("EXL3_GEMV_APPROX"))
 
 def _approx(m: int, mul1: bool) -> bool:
     return bool(GEMV_APPROX) and mul1 and m <= _lib.GEMV_FUSED_MAX_ROWS
+
+
+def _hold(x2: torch.Tensor, mul1: bool) -> bool:
+    """Whether a launch keeps the GEMV up to the boundary against the prefill GEMM: the approximate form
+    that the user asked for, or a stream that captures a graph without the workspace that the
+    register-decode GEMM needs (it would record the unsplit prefill GEMM: gate at 16 rows 64 us, on the
+    GEMV 28)."""
+    m = x2.shape[0]
+    return MID_MR < m <= _lib.GEMV_MAX_ROWS and (_approx(m, mul1) or
+                                                 (x2.is_cuda and E.captures_without_prefill_workspace(x2)))
+
 
 
 _wbuf: dict = {}
@@ -191,7 +201,7 @@ def _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y, gemv: Optional[bool] = 
     M, k = x2.shape
     n = svh.shape[0]
     if gemv is None:
-        gemv = gemv_rows(M, k, n, K, (n,), y.stride(0), _approx(M, mul1))
+        gemv = gemv_rows(M, k, n, K, (n,), y.stride(0), _hold(x2, mul1))
     if gemv and _approx(M, mul1):
         rc = E.exl3_gemv_mr_approx(x2, trellis, y, suh, None, svh, K, GEMV_APPROX)
         if rc != 0:
@@ -270,8 +280,8 @@ def _linear_groups(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch
     # runs of consecutive groups with equal K share one launch, each group written straight into
     # its row-strided column slice; each run takes the route of its own shape (EXL3_GATED=fused: gate and
     # up that of their one-launch form, so that both stay bitwise the same)
-    hold = _approx(M, mul1) or (GATED_ROUTE == "fused" and ng == 2 and K[0] == K[1] and widths[0] == widths[1]
-                                and M <= _lib.GEMV_FUSED_MAX_ROWS)
+    hold = _hold(x2, mul1) or (GATED_ROUTE == "fused" and ng == 2 and K[0] == K[1] and widths[0] == widths[1]
+                               and M <= _lib.GEMV_FUSED_MAX_ROWS)
     i, n0 = 0, 0
     while i < ng:
         j = i + 1
@@ -371,7 +381,7 @@ def exl3_silu_mul_linear(gu: torch.Tensor, trellis: torch.Tensor, suh: torch.Ten
     if M == 0:
         return y.view(*gu.shape[:-1], n)
     approx = _approx(M, mul1)
-    gemv = gemv_rows(M, k, n, K, hold=approx)
+    gemv = gemv_rows(M, k, n, K, hold=_hold(g2, mul1))
     if gemv and M <= _lib.GEMV_FUSED_MAX_ROWS and not approx:
         rc = E.exl3_gemv_silu_in(g2[:, :k], g2[:, k:], trellis, y, suh, None, svh, K, mcg, mul1)
         if rc != 0:

@@ -146,3 +146,49 @@ def test_gated_form_keeps_its_rows(monkeypatch, m):
     fused = m <= 32
     assert calls(torch.ops.exl3rocm.linear_groups) == (["exl3_gemv_mr_grouped"] if fused else ["exl3_gemm_trellis_grouped"])
     assert calls(torch.ops.exl3rocm.linear_silu_mul) == (["exl3_gemv_silu_mul"] if fused else ["exl3_gemm_trellis_grouped", "silu_mul"])
+
+
+# ---------------------------------------------------------------------------------- workspaces and capture
+from exl3rocm import kernels as E  # noqa: E402
+
+CPU = torch.device("cpu")
+
+
+@pytest.fixture
+def workspaces(monkeypatch):
+    """Empty workspace tables, on the CPU."""
+    for name, empty in (("_workspaces", {}), ("_reserved", {}), ("_pf_workspaces", {}), ("_pf_reserved", set())):
+        monkeypatch.setattr(E, name, empty)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+
+
+def test_first_eager_call_brings_both_workspaces(monkeypatch, workspaces):
+    """A layer's reservation at load reaches every stream with its first eager call, whatever its rows; without
+    one a small GEMV call allocates its own workspace only."""
+    E.workspace(CPU, 100, 6)
+    assert list(E._workspaces) == [(CPU, 6)] and not E._pf_workspaces
+    E.reserve_prefill_workspace(CPU, 0)
+    E.workspace(CPU, 5000, 7)
+    assert sorted(s for _, s in E._pf_workspaces) == [0, 7]
+    assert all(b.numel() == E.prefill_workspace_bound() for b in E._pf_workspaces.values())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError):
+        E.workspace(CPU, 100, 8)
+    assert E.prefill_workspace(CPU, 100, 8) is None and (CPU, 8) not in E._pf_workspaces
+
+
+@pytest.mark.parametrize("m,gemv", [(8, True), (9, True), (17, True), (18, False)])
+def test_capture_without_the_prefill_workspace(monkeypatch, m, gemv):
+    """A stream that captures without it keeps the boundary against the prefill GEMM, which is what it would
+    record above."""
+    k, n = 5120, 5120
+    rec = _Mlp()
+    rec.captures_without_prefill_workspace = lambda x: True
+
+    class Input:                                                  # _hold's questions to a GPU tensor
+        shape, is_cuda = (m, k), True
+
+    monkeypatch.setattr(ops, "E", rec)
+    assert ops.gemv_rows(m, k, n, hold=ops._hold(Input, True)) == gemv
+    rec.captures_without_prefill_workspace = lambda x: False
+    assert ops.gemv_rows(m, k, n, hold=ops._hold(Input, True)) == (m <= 8)
