@@ -90,7 +90,7 @@ def prefill_workspace_bound() -> int:
 
 def prefill_workspace(device: torch.device, nbytes: int, stream: Optional[int] = None) -> Optional[torch.Tensor]:
     """Zeroed workspace of the prefill GEMM's split tail and the register-decode GEMM's partial tiles
-    for the current (or given) stream.  A stream's first call outside graph capture allocates the
+    for the current (or given) stream.  A stream's first use outside graph capture allocates the
     size every shape fits in (exl3_gemm_trellis_workspace_max), so a later capture on that stream
     splits exactly as eager calls do.  A stream that captures without one gets None: the ops keep up to
     64 rows on the GEMV there as far as it beats the prefill GEMM (ops.gemv_max_rows), and more rows run the
@@ -109,6 +109,15 @@ def prefill_workspace(device: torch.device, nbytes: int, stream: Optional[int] =
             return buf
         buf = torch.zeros(max(nbytes, prefill_workspace_bound()), dtype=torch.uint8, device=device)
         _pf_workspaces[key] = buf
+    return buf
+
+
+def _launch_workspace(device: torch.device, stream: int, m: int, k: int, wa, groups: int, K: int, ldy: int) -> Optional[torch.Tensor]:
+    """The stream's prefill workspace for a GEMM launch: allocated by the first launch that uses one (split
+    tiles or the register-decode GEMM), so a stream of others never holds its ~45 MB."""
+    buf = _pf_workspaces.get((device, stream))
+    if buf is None and (L.lib().exl3_gemm_rd_serves(m, k, wa, groups, K, ldy) or L.lib().exl3_gemm_trellis_workspace_size(m, k, wa, groups)):
+        buf = prefill_workspace(device, prefill_workspace_bound(), stream)
     return buf
 
 
@@ -398,8 +407,9 @@ def exl3_gemm_trellis_silu_in(gate, up, B, C, suh, xh, svh, K: int, mcg: bool, m
     ldx = g2.stride(0) if m > 1 else k
     wa = (C_int * 1)(n)
     st = _stream(gate)
-    ws = prefill_workspace(gate.device, prefill_workspace_bound(), st)
-    L.check(L.lib().exl3_gemm_trellis_silu_in(g2.data_ptr(), u2.data_ptr(), ldx, B.data_ptr(), C.data_ptr(), _ldy(C, n),
+    ldy = _ldy(C, n)
+    ws = _launch_workspace(gate.device, st, m, k, wa, 1, K, ldy)
+    L.check(L.lib().exl3_gemm_trellis_silu_in(g2.data_ptr(), u2.data_ptr(), ldx, B.data_ptr(), C.data_ptr(), ldy,
                                               suh.data_ptr(), xh.data_ptr(), svh.data_ptr(), m, k, n, K,
                                               *_cb_flags(mcg, mul1), ws.data_ptr() if ws is not None else None,
                                               ws.numel() if ws is not None else 0, st),
@@ -475,9 +485,10 @@ def exl3_gemm_trellis_grouped(A, B: Sequence[torch.Tensor], C, suh: Sequence[tor
     ps, _b = L.ptr_array([s.data_ptr() for s in suh])
     pv, _c = L.ptr_array([s.data_ptr() for s in svh])
     st = _stream(A)
-    ws = prefill_workspace(A.device, prefill_workspace_bound(), st)
+    ldy = _ldy(C, sum(widths))
+    ws = _launch_workspace(A.device, st, m, k, wa, g, K, ldy)
     L.check(L.lib().exl3_gemm_trellis_grouped(x2.data_ptr(), x2.stride(0) if m > 1 else k, pt, C.data_ptr(),
-                                              _ldy(C, sum(widths)), ps, xh.data_ptr(), pv, wa, g, m, k, K,
+                                              ldy, ps, xh.data_ptr(), pv, wa, g, m, k, K,
                                               *_cb_flags(mcg, mul1), ws.data_ptr() if ws is not None else None,
                                               ws.numel() if ws is not None else 0, st),
             "exl3_gemm_trellis_grouped")

@@ -192,3 +192,15 @@ def test_capture_without_the_prefill_workspace(monkeypatch, m, gemv):
     assert ops.gemv_rows(m, k, n, hold=ops._hold(Input, True)) == gemv
     rec.captures_without_prefill_workspace = lambda x: False
     assert ops.gemv_rows(m, k, n, hold=ops._hold(Input, True)) == (m <= 8)
+
+
+def test_launches_that_need_no_workspace_allocate_none(workspaces):
+    def ws(m, k, widths, K=4, stream=5):
+        return E._launch_workspace(CPU, stream, m, k, (ctypes.c_int * len(widths))(*widths), len(widths), K, sum(widths))
+
+    assert ws(300, 512, (512, 384)) is None and ws(2048, 5120, (128 * 256,)) is None and ws(96, 896, (512,)) is None
+    assert not E._pf_workspaces
+    assert ws(256, 1024, (128 * 260,)) is not None                # a split tail
+    first = E._pf_workspaces[(CPU, 5)]
+    assert ws(300, 512, (512,)) is first and ws(20, 5120, (5120,)) is first
+    assert ws(20, 5120, (5120,), stream=6) is not None and len(E._pf_workspaces) == 2   # the register-decode GEMM
