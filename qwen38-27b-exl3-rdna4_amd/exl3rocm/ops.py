@@ -41,25 +41,41 @@ MR_MAX: Optional[int] = _env_rows("EXL3_MR_MAX")
 # the library's comparison knob; set, the register-decode GEMM is not taken
 GEMM_KERNEL = os.environ.get("EXL3_GEMM_KERNEL", "")
 DEFAULT_MR = 32
-MID_MR, MID_K = 8, 3072
-# Largest row count at which the fused GEMV beats the register-decode GEMM, by (k, output columns of the
-# launch: all its groups).  Measured on MI355X for the launches a Qwen3.5-27B checkpoint makes (q/k/v and
-# gate/up grouped as linear_groups groups them, and lm_head) and 4096 x 4096: both routes at 20 row
-# counts from 2 to 64, graphs of 16 launches over cold weights, 4 bpw, and 2 / 3 / 5 bpw where a
-# checkpoint holds them.  The GEMV's cost grows with every row, the register-decode GEMM's (up to
-# 128 rows) only with each 32-row tile: they cross at 8 to 9 rows on every shape (5120 -> 5120 14.4 /
-# 15.1 us at 8 rows, 17.4 / 15.1 at 9; gate 25.8 / 24.8 and 27.3 / 24.7; down 24.2 / 25.4 and 26.6 /
-# 25.4; gate/up 38.4 / 37.7 and 39.6 / 37.8), so 8 rows it is: those stay bitwise equal to their
-# one-row calls on every shape.  (lm_head stays at 32: its rows up to there are used as one-row calls'
-# when drafted tokens are verified.)  Up to 8 bpw and for the mcg / 3inst codebooks alike: both routes
-# run the same decoder.  Shapes outside the table: from 3072 inputs the same 8; below them the default
-# 32, the row count up to which a linear has always been its one-row calls (2048 x 2048 16.9 us against
-# 11.1 at 32 rows, 9.0 against 10.7 at 8).
+# Largest row count of the fused GEMV where the register-decode GEMM serves the launch, by (k, output columns
+# of the launch: all its groups).  The GEMV's cost grows with every row and steps at 17, its second
+# 16-row tile; the GEMM's (up to 128 rows) only with each 32-row tile.  Measured on MI355X, GEMV / GEMM in us,
+# graphs of 16 launches over cold weights, 4 bpw: 5120 -> 5120 14.4 / 15.1 at 8 rows, 17.4 / 15.1 at 9, 26.5 /
+# 15.4 at 20; gate 25.8 / 24.8, 27.3 / 24.7, 36.2 / 26.0; down 24.2 / 25.4, 26.6 / 25.4, 36.5 / 25.6; gate/up
+# 38.4 / 37.7, 39.6 / 37.8, 51.8 / 40.9: the layers' launches of a 27B decoder cross at 8 to 9 rows, and
+# so do other shapes from 3072 to 17408 inputs and 128 to 17408 columns (MID_MR).
+# Where the launch is small the two end within a few us of each other up to the GEMV's step, and a graph
+# of this launch alone pays ~2.3 us for the GEMM's second node, so the GEMV keeps its first 16-row tile
+# (SMALL_MR: up to 2^24 weights of at most 8192 inputs, and either at most 1024 columns or 5 bpw and more,
+# whose pieces take the GEMM longer).  In a graph of 16 / of one launch: 5120 -> 1024 at 4 bpw 13.4 / 14.0 and
+# 17.9 / 19.9 at 9 rows, 14.2 / 13.8 and 18.8 / 19.9 at 16, 17.5 / 14.2 and 21.4 / 20.2 at 20; 4096 -> 4096 at 6 bpw
+# 17.2 / 15.4 and 21.3 / 21.7 at 9, 17.9 / 15.6 and 22.0 / 21.6 at 16, 21.0 / 16.0 and 25.6 / 22.0 at 20.  The k/v
+# pair of 5120 inputs is one of these by the table (15.2 / 14.9 and 19.5 / 20.7 at 10 rows).
+# Two boundaries are there for their rows, which are bitwise their one-row calls, and not for speed: lm_head's
+# 32 rows (216 / 222 us at 9, 229 / 221 at 16, 300 / 232 at 32), and DEFAULT_MR, the boundary of the library's
+# own dispatcher exl3_gemm, below 3072 inputs (2048 -> 2048 11.1 / 11.4 at 9, 16.8 / 11.9 at 32); it is the
+# prefill GEMM's too where k is no multiple of 256.
+MID_MR, MID_K, SMALL_MR = 8, 3072, 16
 GEMV_CROSSOVER = {
-    (5120, 1024): 8, (5120, 2048): 8, (5120, 5120): 8, (5120, 6144): 8, (5120, 7168): 8,
+    (5120, 1024): 16, (5120, 2048): 16, (5120, 5120): 8, (5120, 6144): 8, (5120, 7168): 8,
     (5120, 10240): 8, (5120, 12288): 8, (5120, 14336): 8, (5120, 16384): 8, (5120, 17408): 8,
     (5120, 34816): 8, (5120, 248320): 32, (6144, 5120): 8, (17408, 5120): 8,
 }
+
+
+def _crossover(k: int, width: int, K: int) -> int:
+    b = GEMV_CROSSOVER.get((k, width))
+    if b is not None:
+        return b
+    if k < MID_K or k % 256:
+        return DEFAULT_MR
+    return SMALL_MR if k * width <= 1 << 24 and k <= 8192 and (width <= 1024 or K >= 5) else MID_MR
+
+
 # The same against the prefill GEMM (other shapes: DEFAULT_MR), for launches that the register-decode GEMM
 # does not serve: both routes at every row count from 2 to 64, graphs of 24 launches over 8 weight
 # copies, 4 bpw, and 2 / 3 bpw where a checkpoint holds them (the boundary moved by <= 4 rows).  Each
@@ -91,7 +107,7 @@ def gemv_max_rows(k: int, width: int, K: int = 4, widths: Optional[tuple] = None
     if hold or PREFILL_ROUTE == "recon" or GEMM_KERNEL or not _rd_serves(k, widths or (width,), K, ldy or width):
         b = PREFILL_CROSSOVER.get((k, width), DEFAULT_MR)
     else:
-        b = GEMV_CROSSOVER.get((k, width), MID_MR if k >= MID_K and k % 256 == 0 else DEFAULT_MR)
+        b = _crossover(k, width, K)
     return min(b, _lib.GEMV_MAX_ROWS)
 
 
@@ -99,8 +115,6 @@ def gemv_rows(m: int, k: int, width: int, K: int = 4, widths: Optional[tuple] = 
               hold: bool = False) -> bool:
     """Route of an m-row launch: the fused GEMV (True; every row bitwise equal to its m = 1 call)
     or a GEMM."""
-    if MR_MAX is None and m <= MID_MR:                        # no boundary is lower
-        return True
     return m <= gemv_max_rows(k, width, K, widths, ldy, hold)
 
 
@@ -138,14 +152,19 @@ def _approx(m: int, mul1: bool) -> bool:
     return bool(GEMV_APPROX) and mul1 and m <= _lib.GEMV_FUSED_MAX_ROWS
 
 
+def _few(m: int) -> bool:
+    """Rows below every boundary: the GEMV without another question (an eager call's host time)."""
+    return MR_MAX is None and m <= MID_MR
+
+
 def _hold(x2: torch.Tensor, mul1: bool) -> bool:
     """Whether a launch keeps the GEMV up to the boundary against the prefill GEMM: the approximate form
     that the user asked for, or a stream that captures a graph without the workspace that the
     register-decode GEMM needs (it would record the unsplit prefill GEMM: gate at 16 rows 64 us, on the
     GEMV 28)."""
     m = x2.shape[0]
-    return MID_MR < m <= _lib.GEMV_MAX_ROWS and (_approx(m, mul1) or
-                                                 (x2.is_cuda and E.captures_without_prefill_workspace(x2)))
+    return m <= _lib.GEMV_MAX_ROWS and (_approx(m, mul1) or
+                                        (x2.is_cuda and E.captures_without_prefill_workspace(x2)))
 
 
 
@@ -201,7 +220,7 @@ def _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y, gemv: Optional[bool] = 
     M, k = x2.shape
     n = svh.shape[0]
     if gemv is None:
-        gemv = gemv_rows(M, k, n, K, (n,), y.stride(0), _hold(x2, mul1))
+        gemv = _few(M) or gemv_rows(M, k, n, K, (n,), y.stride(0), _hold(x2, mul1))
     if gemv and _approx(M, mul1):
         rc = E.exl3_gemv_mr_approx(x2, trellis, y, suh, None, svh, K, GEMV_APPROX)
         if rc != 0:
@@ -280,15 +299,16 @@ def _linear_groups(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch
     # runs of consecutive groups with equal K share one launch, each group written straight into
     # its row-strided column slice; each run takes the route of its own shape (EXL3_GATED=fused: gate and
     # up that of their one-launch form, so that both stay bitwise the same)
-    hold = _hold(x2, mul1) or (GATED_ROUTE == "fused" and ng == 2 and K[0] == K[1] and widths[0] == widths[1]
-                               and M <= _lib.GEMV_FUSED_MAX_ROWS)
+    few = _few(M)
+    hold = few or _hold(x2, mul1) or (GATED_ROUTE == "fused" and ng == 2 and K[0] == K[1] and widths[0] == widths[1]
+                                     and M <= _lib.GEMV_FUSED_MAX_ROWS)
     i, n0 = 0, 0
     while i < ng:
         j = i + 1
         while j < ng and j - i < _lib.MAX_GROUPS and K[j] == K[i]:
             j += 1
         w = sum(widths[i:j])
-        gemv = gemv_rows(M, k, w, K[i], tuple(widths[i:j]), y.stride(0), hold)
+        gemv = few or gemv_rows(M, k, w, K[i], tuple(widths[i:j]), y.stride(0), hold)
         if j == i + 1 or (gemv and _approx(M, mul1)) or \
                 (not gemv and PREFILL_ROUTE == "recon"):
             # one group, the approximate GEMV or the recon prefill: each group its own launch
@@ -381,7 +401,7 @@ def exl3_silu_mul_linear(gu: torch.Tensor, trellis: torch.Tensor, suh: torch.Ten
     if M == 0:
         return y.view(*gu.shape[:-1], n)
     approx = _approx(M, mul1)
-    gemv = gemv_rows(M, k, n, K, hold=_hold(g2, mul1))
+    gemv = _few(M) or gemv_rows(M, k, n, K, hold=_hold(g2, mul1))
     if gemv and M <= _lib.GEMV_FUSED_MAX_ROWS and not approx:
         rc = E.exl3_gemv_silu_in(g2[:, :k], g2[:, k:], trellis, y, suh, None, svh, K, mcg, mul1)
         if rc != 0:

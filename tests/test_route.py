@@ -22,12 +22,24 @@ def defaults(monkeypatch):
 
 
 def test_boundaries():
-    """No boundary below MID_MR (gemv_rows answers those rows at once), none against the prefill GEMM
+    """No boundary below MID_MR (the ops ask nothing at those rows), none against the prefill GEMM
     below the one against the register-decode GEMM, which starts to win earlier."""
     assert sorted(ops.PREFILL_CROSSOVER) == CHECKPOINT
     for s in CHECKPOINT:
         assert ops.MID_MR <= ops.GEMV_CROSSOVER[s] <= ops.PREFILL_CROSSOVER[s] <= _lib.GEMV_MAX_ROWS
     assert ops.MID_MR <= ops.DEFAULT_MR
+
+
+def test_small_launches():
+    """Launches of at most 2^24 weights that the register-decode GEMM does not speed up keep the GEMV's
+    first 16-row tile; neighbours on each side of the rule do not."""
+    for k, w, K in ((4096, 4096, 6), (4096, 4096, 5), (3072, 128, 4), (8192, 1024, 1), (5120, 1024, 4), (5120, 2048, 4), (3072, 5376, 8)):
+        assert ops.gemv_max_rows(k, w, K) == 16, (k, w, K)
+    for k, w, K in ((4096, 4096, 4), (4096, 4224, 6), (3072, 1152, 4), (8448, 1024, 8), (12288, 128, 4), (5120, 5120, 8)):
+        assert ops.gemv_max_rows(k, w, K) == 8, (k, w, K)
+    for k, w in ((2048, 2048), (3072 + 128, 1024), (2816, 128)):
+        assert ops.gemv_max_rows(k, w, 8) == ops.DEFAULT_MR
+    assert ops.gemv_rows(16, 4096, 4096, 6) and not ops.gemv_rows(17, 4096, 4096, 6)
 
 
 @pytest.mark.parametrize("knob,value", [("PREFILL_ROUTE", "recon"), ("GEMM_KERNEL", "tile"), ("GEMM_KERNEL", "pc")])
