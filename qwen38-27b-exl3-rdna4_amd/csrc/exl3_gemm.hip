@@ -894,13 +894,16 @@ int launch_trellis_gemm(const uint16_t* const* xh, int64_t ldx, const void* cons
     a.xcd_remap = a.n_full % 8 == 0;
     if (pl.split > 1) {
         // the tiles' counters as far apart as the head has room for (a power of two of words, at most
-        // two 128-byte lines; split tiles: at most 170, 128 of three or more pieces): the polls of
-        // many tiles on one line delayed the other pieces' partials by 4 to 8 us
+        // two 128-byte lines): the polls of many tiles on one line delayed the other pieces' partials by
+        // 4 to 8 us.  Tiles of three or more pieces need two words each.
+        static_assert((2 * PC_CUS / 3) * 4 <= (int) PC_COUNTER_BYTES, "one word for each of at most 170 tiles of two pieces");
+        static_assert((PC_CUS / 3) * 8 <= (int) PC_COUNTER_BYTES, "two words for each of at most 85 tiles of more");
         a.counters = (uint32_t*) ws;
-        const char* ep = getenv("EXL3_GEMM_POLLS");          // (tests: 0, nobody waits)
+        const char* ep = e && e[0] ? getenv("EXL3_GEMM_POLLS") : nullptr;   // (tests: 0, nobody waits)
         a.polls = ep ? std::min(std::max(atoi(ep), 0), PC::POLLS) : PC::POLLS;
         a.cstride = 64;
         while (a.cstride * (tiles - a.n_full) * 4 > (int) PC_COUNTER_BYTES) a.cstride /= 2;
+        if (a.cstride < (a.split > 2 ? 2 : 1)) return EXL3_EINVAL;          // (no plan has it)
         a.part = (f32x4*) ((char*) ws + PC_COUNTER_BYTES);
         a.part_bytes = (uint32_t) (pl.ws_bytes - PC_COUNTER_BYTES);
     }

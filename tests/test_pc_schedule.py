@@ -203,3 +203,22 @@ def test_unequal_pieces_plan_matches_the_library():
     assert pc_steps_of_plan(33, 5120, [17408]) == {80, 54, 26}
     assert ws(33, 5120, [17408 + 128 * 60]) == 0                 # 196 tiles: unsplit, no workspace
     assert ws(33, 5120, [128 * 100]) == 4096 + 100 * 2 * piece   # 100 tiles: 2 equal pieces (min(256 / 100, 10))
+
+
+def test_counters_fit_the_workspace_head():
+    """Tiles of three or more pieces have two counters each (at most 85 such tiles), tiles of two pieces
+    one (at most 170), in the 4 KB head: every plan of 1 to 600 tiles, from the workspace the library asks for."""
+    import ctypes
+    from exl3rocm import _lib
+    L = _lib.lib()
+    most = {2: 0, 3: 0}
+    for tiles in range(1, 601):
+        for k in (1024, 1792, 5120, 17408):
+            b = L.exl3_gemm_trellis_workspace_size(256, k, (ctypes.c_int * 1)(128 * tiles), 1)
+            tail = tiles % 256
+            if b:
+                assert (b - 4096) % (256 * 128 * 4) == 0 and (b - 4096) // (256 * 128 * 4) % tail == 0
+                split = (b - 4096) // (256 * 128 * 4) // tail
+                most[min(split, 3)] = max(most[min(split, 3)], tail)
+    assert most == {2: 170, 3: 85}
+    assert most[2] * 4 <= 4096 and most[3] * 8 <= 4096
