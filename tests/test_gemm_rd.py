@@ -96,7 +96,7 @@ CASES = [  # m, k, widths, bits, cb
     (9, 5120, [5120], 4, 2), (31, 2048, [128], 1, 0), (32, 2304, [384], 2, 1), (33, 2048, [256, 128], 3, 2),
     (63, 4096, [512], 5, 0), (64, 5120, [1024, 1024], 6, 1), (65, 2560, [640], 7, 2), (96, 3072, [256], 8, 0),
     (97, 2048, [1024, 128, 128], 4, 1), (127, 5120, [256], 3, 0), (128, 2048, [384], 8, 2), (1, 2048, [256], 5, 1),
-    (40, 2048, [128 * 260], 2, 2),          # more tiles than workgroups: pieces cross tiles, whole tiles between
+    (40, 2048, [128 * 260], 2, 2),          # more tiles than workgroups: pieces cross tiles, next to whole tiles
     (100, 5120, [17408], 4, 2),             # 136 tiles in 256 pieces that cross them
     (48, 17408, [768], 3, 2),
 ]
@@ -117,6 +117,56 @@ def test_against_the_oracle(m, k, widths, bits, cb):
     for (tr, su, sv), n in zip(mats, widths):
         assert_close(y[rows, n0:n0 + n].cpu().numpy(), cpu.linear(x[rows], tr, bits, su, sv, cb), (m, k, n0))
         n0 += n
+
+
+def segments(tiles, upt, G=256):
+    """Each workgroup's segments where pieces cross tiles: [(tile, whole)], of an even share of the units."""
+    out = []
+    for c in range(G):
+        u, end, seg = tiles * upt * c // G, tiles * upt * (c + 1) // G, []
+        while u < end:
+            t = u // upt
+            stop = min(end, (t + 1) * upt)
+            seg.append((t, u == t * upt and stop == (t + 1) * upt))
+            u = stop
+        out.append(seg)
+    return out
+
+
+WIDE = 700                                                        # tiles of 8 units in 256 workgroups
+
+
+def test_wide_launch_has_every_segment_order():
+    """What the next test runs: a shared first tile, one or two whole tiles, a shared last one, and each of
+    these orders without its first or last."""
+    orders = {"".join("W" if w else "P" for _, w in seg) for seg in segments(WIDE, 8)}
+    assert orders == {"WWP", "PWP", "PWWP", "PWW"}
+    assert check(20, 2048, [128 * WIDE]) == 0
+
+
+@gpu
+@needs_gpu
+@pytest.mark.parametrize("m", [20, 40, 80, 128])                  # one case for each count of row tiles
+def test_whole_tiles_between_shared_ones(m):
+    """Every tile of a launch of 700 against the unsplit prefill GEMM, and the tiles of workgroups that
+    have whole tiles between shared ones against the oracle."""
+    k, n, bits, cb = 2048, 128 * WIDE, 1, 2
+    print(f"register-decode whole tiles between m={m}", flush=True)
+    x, mats, X, (T, SU, SV) = module("rd-wide", k, [n], bits, m)
+    y, again = grouped(X, T, SU, SV, bits, cb), grouped(X, T, SU, SV, bits, cb)
+    want = torch.empty_like(y)
+    E.exl3_gemm_trellis(X, T[0], want, SU[0], torch.empty_like(X), SV[0], bits, False, True)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), again.view(torch.int16))
+    # two routes, each within the bar (rel-L2 1e-3) of the oracle: 2e-3 of each other, tile by tile
+    d, w = ((v.double().view(m, WIDE, 128) ** 2).sum((0, 2)).sqrt() for v in (y.double() - want.double(), want))
+    assert bool((d <= 2e-3 * w).all()), [int(t) for t in (~(d <= 2e-3 * w)).nonzero()[:8]]
+    tr, su, sv = mats[0]
+    rows = sorted({0, min(m - 1, 31), min(m - 1, 32), m - 1})
+    for seg in [g for g in segments(WIDE, 8) if len(g) >= 3][::80]:
+        c0, c1 = 128 * seg[0][0], 128 * (seg[-1][0] + 1)
+        ref = cpu.linear(x[rows], np.ascontiguousarray(tr[:, c0 // 16:c1 // 16]), bits, su, np.ascontiguousarray(sv[c0:c1]), cb)
+        assert_close(y[rows, c0:c1].cpu().numpy(), ref, (m, seg))
 
 
 @gpu
