@@ -14,7 +14,7 @@ import torch
 
 import cpu
 import isa_waits as W
-from exl3rocm import _lib, kernels as E, synth
+from exl3rocm import _lib, kernels as E, ops, synth
 
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(REPO, "qwen38-27b-exl3-rdna4_amd", "exl3rocm", "libexl3_mi355x.so")
@@ -195,10 +195,26 @@ def test_rows_do_not_interact_and_strides():
 
 @gpu
 @needs_gpu
+def test_rows_are_the_same_in_every_batch():
+    """A row's bits do not depend on the batch: up to 64 rows (exact transforms), and from 65 (float32 ones).
+    The split of the work is by shape alone and every row is summed in the same order."""
+    k, widths, bits = 5120, [640, 128], 4
+    x, mats, X, (T, SU, SV) = module("rd-batch", k, widths, bits, 128)
+    y64, y128 = grouped(X[:64], T, SU, SV, bits, 2), grouped(X, T, SU, SV, bits, 2)
+    for m in (1, 9, 32, 33):
+        assert torch.equal(grouped(X[:m], T, SU, SV, bits, 2).view(torch.int16), y64[:m].view(torch.int16)), m
+    for m in (65, 97):
+        assert torch.equal(grouped(X[:m], T, SU, SV, bits, 2).view(torch.int16), y128[:m].view(torch.int16)), m
+
+
+@gpu
+@needs_gpu
 @pytest.mark.parametrize("m", [20, 90])
 def test_silu_input_and_graph_replays(m):
     """The SiLU-input form equals silu_mul and the plain form bitwise; replays of a captured call equal
     the eager one, eager work between them."""
+    if ops.PREFILL_ROUTE != "fused" or ops.GEMM_KERNEL or ops.MR_MAX is not None:
+        pytest.skip("a knob chooses the route")
     k, n, bits = 4096, 768, 4
     x, mats, X, (T, SU, SV) = module("rd-silu", k, [n], bits, m)
     gu = torch.cat([X, X.flip(0)], 1).contiguous()

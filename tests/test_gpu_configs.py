@@ -394,6 +394,8 @@ def test_routing_follows_the_measured_crossover(k, widths, bits):
     last rows of both against the oracle."""
     if ops.PREFILL_ROUTE != "fused":
         pytest.skip("EXL3_PREFILL selects the reconstruct + GEMM route above the boundary")
+    if ops.GEMM_KERNEL or (ops.GATED_ROUTE == "fused" and len(widths) == 2):
+        pytest.skip("a knob keeps the boundary against the prefill GEMM")
     b = ops.gemv_max_rows(k, sum(widths))
     assert ops.MR_MAX is None and b == ops.GEMV_CROSSOVER[(k, sum(widths))]
     g = len(widths)
