@@ -4,8 +4,11 @@
 // launches, the input transform (launch_had, in fragment order) and this kernel.
 //
 // What bounds it.  Every weight is decoded once, ~4 vector instructions a weight whatever the rows (the
-// GEMV's bound too), and the matrix cores' share grows with R: 137 + ~20 vector and 4 R matrix
-// instructions (32 cycles each) per 32 k x 64 columns and wave.  The 256-row prefill kernel pays its LDS
+// GEMV's bound too), and the matrix cores' share grows with R: 141 / 156 / 152 / 160 vector (R = 1 to 4; the
+// whole kernel's count over its loop's steps) and 4 R matrix instructions (32 cycles each) per 32 k x 64
+// columns and wave.  The two hardly overlap: counted at gate/up 5120 -> 2 x 17408, 4 bpw, vector issue takes
+// 70 / 65 / 54 / 49 % of a busy CU's cycles and the matrix cores 16 / 27 / 35 / 40 % at 32 / 64 / 96 / 128 rows,
+// 86 to 92 % together.  The 256-row prefill kernel pays its LDS
 // round trip of the weights and a barrier per 64 k for rows that are not there (gate 5120 -> 17408: 1.1
 // us a step, 60 us, at 64 rows as at 256).  Here a wave keeps what it decodes:
 //   * a lane's q-block is a 32x32x16 MFMA's B operand as it stands (lane bit 5: k-tile, bits 4..0:
@@ -21,9 +24,8 @@
 // Measured (4 bpw, graphs of 16 launches over cold weights, transform included; before: the faster of
 // GEMV and prefill GEMM): gate/up 5120 -> 2 x 17408 at 16 / 32 / 64 / 96 / 128 rows 42 / 57 / 89 / 113 /
 // 118 -> 38 / 40 / 53 / 65 / 79 us; gate 29 / 41 / 60 / 65 / 67 -> 25 / 26 / 34 / 43 / 51; 5120 -> 5120 19 /
-// 26 / 34 / 36 / 37 -> 15 / 16 / 21 / 25 / 28; at 32 rows the loop runs ~0.34 us a wave's 32 k x 64 columns
-// (86 % of the vector issue rate), the other ~13 us are the transform's launch, the first loads and the
-// completion.
+// 26 / 34 / 36 / 37 -> 15 / 16 / 21 / 25 / 28; at 32 rows such a step takes a SIMD 0.37 us (gate/up's 85 of
+// them against 5120 -> 5120's 20), the other ~9 us are the transform's launch, the first loads and the completion.
 #include "exl3_gemm_rd.h"
 
 #include <algorithm>
@@ -563,8 +565,9 @@ int launch_rd_cb(int cb, int R, const RdArgs& a, int grid, hipStream_t s)
 RdPlan rd_plan(int M, int K, const int* widths, int groups)
 {
     RdPlan p{};
-    // K below 2048 stays with the prefill kernel: its launches too short to split are bitwise equal to
-    // reconstruct + hgemm and between grouped and single calls, which cut tiles are not
+    // K below 2048 (at most 7 units a tile) stays with the prefill kernel.  Below 1024 that never splits a
+    // tile, so its launches are bitwise equal to reconstruct + hgemm and between grouped and single calls,
+    // which cut tiles are not; from 1024 to 2047 this kernel was not measured
     if (M < 1 || M > RD_MAX_ROWS || K % 256 || K < 2048) return p;
     // the rotated input of a group is read through a raw buffer with 32-bit byte offsets
     if ((uint64_t) M * (uint64_t) K * 2 >= (1ull << 31)) return p;
