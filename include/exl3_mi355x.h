@@ -79,8 +79,8 @@ int exl3_had_r_128(const void* in, int64_t ld_in, void* out, int64_t ld_out, int
  * at most the error of an fp32 summation of a block's 128 terms before that rounding).  (The fused
  * GEMV's transforms are float64, exl3_had_r_128's values.)
  * No counterpart of its own in the reference (whose had_r_128 serves both roles, ops.py:88,97).
- * Callers: exl3rocm's reconstruct + hgemm_recon prefill route, so that it stays bitwise equal to
- * the fused prefill route. */
+ * Callers: exl3rocm's reconstruct + hgemm_recon prefill route, so that it is bitwise equal to
+ * the fused route wherever that is the prefill GEMM with whole tiles. */
 int exl3_had_r_128_f32(const void* in, int64_t ld_in, void* out, int64_t ld_out, int rows, int cols, const void* pre,
                        const void* post, float scale, void* stream);
 
@@ -214,7 +214,7 @@ int exl3_gemv_silu_mul(const void* x, int64_t ldx, const void* const* trellis, v
 /* Elementwise SiLU-and-mul: out[r][c] = fp16(fp16(silu(gate[r][c])) * up[r][c]) for r < rows,
  * c < n (n % 8 == 0; gate and up rows ld_in apart, out rows ld_out apart; 16-byte aligned).
  * No counterpart in the reference (vLLM's SiluAndMul does this there).  Callers: exl3rocm's
- * linear_silu_mul op for m > 32, after the grouped prefill. */
+ * linear_silu_mul op, after the gate and up linears. */
 int exl3_silu_mul(const void* gate, const void* up, int64_t ld_in, void* out, int64_t ld_out, int rows, int n,
                   void* stream);
 
@@ -243,8 +243,9 @@ int exl3_hgemm_recon(const void* x, int64_t ldx, const void* W, int64_t ldw, voi
                      void* stream);
 
 /* Prefill EXL3 linear for any m: the trellis is decoded into LDS tiles and fed to fp16 MFMA
- * with fp32 accumulation; input and output Hadamards run as separate passes.  xh is an
- * [m, k] fp16 scratch (the rotated input).
+ * with fp32 accumulation; the input Hadamard is a pass of its own.  xh is an [m, k] fp16 scratch (the
+ * rotated input).  It has no workspace, so it is the prefill GEMM with whole tiles at every m: up to
+ * 256 rows are mostly faster through exl3_gemm_trellis_grouped with one group and a workspace.
  * Replaces the reconstruct + hgemm_recon route of `exl3rocm::linear` (reference ops.py:86-97). */
 int exl3_gemm_trellis(const void* x, int64_t ldx, const void* trellis, void* y, int64_t ldy, const void* suh,
                       void* xh, const void* svh, int m, int k, int n, int K, int mcg, int mul1, void* stream);
@@ -252,10 +253,13 @@ int exl3_gemm_trellis(const void* x, int64_t ldx, const void* trellis, void* y, 
 /* Prefill EXL3 linear of up to 4 groups sharing x and K but of any widths (the checkpoint tensors
  * of a fused module: q / k / v, gate / up): group i writes the widths[i] columns of y that follow
  * groups 0 .. i-1 (rows ldy apart, ldy >= sum of widths).  xh is an fp16 scratch of groups * m * k
- * elements (each group's rotated input).  No counterpart in the reference: its linear_groups runs
+ * elements (each group's rotated input, in the order that the kernel reads: not a result).  With
+ * exl3_gemm_trellis_workspace_max() bytes of workspace up to 128 rows run on the register-decode GEMM
+ * where exl3_gemm_rd_serves says so (exact transforms up to 64 rows, float32 ones above; a row's bits
+ * are the same in every batch of up to 64 rows, and of 65 to 128); everything else on the prefill GEMM.  No counterpart in the reference: its linear_groups runs
  * one prefill per group (reference vllm_plugin/exl3rocm/ops.py:171-175).  Callers: exl3rocm's
- * linear_groups for M > 32.  All groups' output tiles share one GEMM launch, so a module fills the
- * GPU as one layer would.  workspace / ws_bytes: see exl3_gemm_trellis_workspace_size. */
+ * ops above the GEMV's rows.  All groups' output tiles share one GEMM launch, so a module fills the
+ * GPU as one layer would.  workspace / ws_bytes: see exl3_gemm_trellis_workspace_max. */
 int exl3_gemm_trellis_grouped(const void* x, int64_t ldx, const void* const* trellis, void* y, int64_t ldy,
                               const void* const* suh, void* xh, const void* const* svh, const int* widths, int groups,
                               int m, int k, int K, int mcg, int mul1, void* workspace, size_t ws_bytes,
@@ -265,31 +269,31 @@ int exl3_gemm_trellis_grouped(const void* x, int64_t ldx, const void* const* tre
  * prefill of one group over the input x = fp16(fp16(silu(gate)) * up) (the exl3_silu_mul
  * roundings), formed by the input transform as it loads the rows; gate and up rows ldx apart (a
  * gated module's grouped [m, 2k] output: gate = y, up = y + k, ldx = 2k).  xh: [m, k] fp16
- * scratch (the rotated activation); workspace / ws_bytes: exl3_gemm_trellis_workspace_size(m, k,
- * &n, 1).  Bitwise equal to exl3_silu_mul followed by exl3_gemm_trellis_grouped.  No counterpart in
+ * scratch; workspace / ws_bytes as exl3_gemm_trellis_grouped.  Bitwise equal to exl3_silu_mul followed by exl3_gemm_trellis_grouped.  No counterpart in
  * the reference: its down projection reads the SiluAndMul output (reference
  * docs/EFFICIENCY_INVESTIGATION.md:36-66 proposes fusing the activation).  Callers: exl3rocm's
- * silu_mul_linear op for m > 32.  Removes the activation launch and its [m, k] write and read. */
+ * silu_mul_linear op above the GEMV's rows.  Removes the activation launch and its [m, k] write and read. */
 int exl3_gemm_trellis_silu_in(const void* gate, const void* up, int64_t ldx, const void* trellis, void* y, int64_t ldy,
                               const void* suh, void* xh, const void* svh, int m, int k, int n, int K, int mcg, int mul1,
                               void* workspace, size_t ws_bytes, void* stream);
 
-/* Workspace bytes exl3_gemm_trellis_grouped uses to balance the launch's last, partial wave of
+/* Workspace bytes the prefill GEMM of exl3_gemm_trellis_grouped uses to balance the launch's last, partial wave of
  * output tiles (those tiles are split along K; fp32 partials and completion counters).  0 when the
  * shape needs none.  Zero before the first call; every call leaves its counters zero.  With a
  * smaller or NULL workspace the tail is not split: the same results to the tolerance, less
- * balance.  No reference counterpart (the reference prefill has no split). */
+ * balance.  Up to 128 rows the register-decode GEMM needs exl3_gemm_trellis_workspace_max() bytes instead.
+ * No reference counterpart (the reference prefill has no split). */
 size_t exl3_gemm_trellis_workspace_size(int m, int k, const int* widths, int groups);
 
 /* The largest workspace exl3_gemm_trellis_workspace_size returns for any shape (a plan splits at
  * most two thirds of one wave of tiles into two pieces, or fewer tiles into at most one wave of
- * pieces): one workspace of this size serves every prefill call, so a caller that reserves it on a
- * stream at load time never needs another before graph capture there.  No reference counterpart.
- * Callers: exl3rocm's prefill workspace. */
+ * pieces): one workspace of this size serves every launch of the prefill GEMM.  No reference
+ * counterpart.  Callers: exl3_gemm_trellis_workspace_max is this and the counters behind it. */
 size_t exl3_gemm_trellis_workspace_bound(void);
 
 /* The workspace with which exl3_gemm_trellis_grouped and exl3_gemm_trellis_silu_in take their fastest
- * plan for every shape: exl3_gemm_trellis_workspace_bound() bytes (split prefill tiles, or the
+ * plan for every shape (a caller that reserves it on a stream at load time never needs another before
+ * graph capture there): exl3_gemm_trellis_workspace_bound() bytes (split prefill tiles, or the
  * register-decode GEMM's partial tiles, up to 128 rows), then that GEMM's completion counters.  Zero
  * before the first call; every call leaves its counters zero.  With a smaller workspace up to 128
  * rows take the prefill GEMM: the same results to the tolerance.  No reference counterpart.

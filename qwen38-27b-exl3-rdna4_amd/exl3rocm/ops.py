@@ -4,16 +4,17 @@ each call as one node.  Same op names, schemas and routing contract as the refer
 ops (vllm_plugin/exl3rocm/ops.py:65-180); kernels come from libexl3_mi355x.so.
 
 One call computes one checkpoint tensor ("group"): y = had(had(x * suh) @ W_inner) * svh.
-Routing by rows M, per launch (gemv_rows: the measured GEMV / GEMM crossover of the launch's shape,
-or EXL3_MR_MAX rows for every shape when set):
+Routing by rows M, per launch (gemv_rows: the measured GEMV / GEMM crossover of the launch's shape, 8 to
+32 rows, or EXL3_MR_MAX rows for every shape when set):
   M <= the crossover     -> fused GEMV (input Hadamard, trellis decode + MFMA dot, split-K
                             reduction and output Hadamard in one launch); every row is bitwise
                             equal to the M == 1 call of that row; EXL3_GEMV_APPROX=affine|int8
                             selects the opt-in approximate mul1 forms (unrounded weights, or
                             int8 activations as the reference's EXL3_ROCM_GFX1201_INT8 path)
   otherwise              -> input Hadamard pass, then a GEMM launch (fp16 MFMA, fp32 accumulate, output
-                            Hadamard and svh in its epilogue): up to 128 rows the register-decode GEMM,
-                            above the prefill GEMM (trellis decoded into LDS);
+                            Hadamard and svh in its epilogue): up to 128 rows the register-decode GEMM
+                            (k from 2048 in multiples of 256), else the prefill GEMM (trellis decoded
+                            into LDS);
                             a fused module's groups share one GEMM launch; EXL3_PREFILL=recon takes
                             the reference's reconstruct + hgemm route instead
 """
@@ -230,7 +231,7 @@ def _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y, gemv: Optional[bool] = 
         if rc != 0:
             raise RuntimeError(f"exl3rocm: GEMV declined shape m={M} k={k} n={n} K={K}")
     elif PREFILL_ROUTE == "recon":
-        # the fused prefill's float32 transforms (exact=False): this route stays bitwise equal to it
+        # the prefill GEMM's float32 transforms (exact=False): this route is bitwise equal to its whole tiles
         xh = torch.empty_like(x2)
         E.had_r_128(x2, xh, suh, None, 1.0, exact=False)
         for n0 in range(0, n, RECON_SLICE_N):
@@ -351,9 +352,9 @@ def exl3_linear_silu_mul(x: torch.Tensor, trellis: list[torch.Tensor], suh: list
     a separate SiluAndMul (the fusion is proposed in reference docs/EFFICIENCY_INVESTIGATION.md:36-66).
 
     Routes: linear_groups, then an elementwise SiLU-and-mul kernel (the default: measured faster
-    on MI355X); or, with EXL3_GATED=fused on the GEMV route (<= 32 rows), equal K and width, one GEMV launch
-    whose workgroup completing a 128-column block of both groups applies the activation.  Both
-    routes give bitwise the same result."""
+    on MI355X); or, with EXL3_GATED=fused up to 32 rows (and the boundary against the prefill GEMM), equal K
+    and width, one GEMV launch whose workgroup completing a 128-column block of both groups applies the
+    activation: bitwise what linear_groups, on the GEMV at those rows under the knob, and SiLU-and-mul give."""
     if not (len(trellis) == 2 and len(suh) == 2 and len(svh) == 2 and len(K) == 2):
         raise RuntimeError("exl3rocm: linear_silu_mul takes exactly two groups (gate, up)")
     n = svh[0].shape[0]

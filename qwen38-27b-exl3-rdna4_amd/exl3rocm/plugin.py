@@ -325,8 +325,8 @@ class Exl3LinearMethod(LinearMethodBase):
             k = layer.exl3_trellis_0.shape[0] * 16
             for K, n in zip(layer.exl3_K, layer.exl3_n):
                 ops.reserve_workspace(dev, k, n, K, groups=min(ng, 4))
-            # the prefill's split workspace: one size serves every shape (each further stream
-            # allocates it on its first eager prefill call)
+            # the GEMMs' workspace: one size serves every shape (each further stream gets its own with
+            # its first eager call)
             ops.E.reserve_prefill_workspace(dev)
             if ops.PREFILL_ROUTE == "recon":
                 ops.reserve_weight_buffer(dev, k * min(max(layer.exl3_n), ops.RECON_SLICE_N))
@@ -363,7 +363,7 @@ class Exl3LinearMethod(LinearMethodBase):
         """The layer's linear of act = fp16(fp16(silu(gate)) * up), gate_up = [gate | up] (the
         [*, 2k] output of the MLP's gate/up module): what `apply(layer, act_fn(gate_up))` gives with
         vLLM's SiluAndMul, bitwise, as one op (exl3rocm::silu_mul_linear: the GEMV or the
-        prefill's input transform forms act as it loads, so act is never written).  No counterpart
+        GEMM's input transform forms act as it loads, so act is never written).  No counterpart
         in the reference plugin, whose MLP runs SiluAndMul and then the down linear.  For MLP code
         that owns both steps; the layer holds one group (a down projection).  Like `apply`, this
         is the local product only: a row-parallel caller still reduces across ranks."""
