@@ -129,8 +129,8 @@ def reserve_prefill_workspace(device: torch.device, stream: Optional[int] = None
 
 
 def captures_without_prefill_workspace(x: torch.Tensor) -> bool:
-    """Whether the current stream captures a graph and has no prefill workspace."""
-    return x.is_cuda and torch.cuda.is_current_stream_capturing() and (x.device, _stream(x)) not in _pf_workspaces
+    """Whether the current stream (of the GPU of x) captures a graph and has no prefill workspace."""
+    return torch.cuda.is_current_stream_capturing() and (x.device, _stream(x)) not in _pf_workspaces
 
 
 def gemv_workspace_bytes(m: int, k: int, n: int, K: int, groups: int = 1) -> int:

@@ -153,20 +153,30 @@ def _approx(m: int, mul1: bool) -> bool:
     return bool(GEMV_APPROX) and mul1 and m <= _lib.GEMV_FUSED_MAX_ROWS
 
 
-def _few(m: int) -> bool:
-    """Rows below every boundary: the GEMV without another question (an eager call's host time)."""
-    return MR_MAX is None and m <= MID_MR
-
-
 def _hold(x2: torch.Tensor, mul1: bool) -> bool:
     """Whether a launch keeps the GEMV up to the boundary against the prefill GEMM: the approximate form
     that the user asked for, or a stream that captures a graph without the workspace that the
     register-decode GEMM needs (it would record the unsplit prefill GEMM: gate at 16 rows 64 us, on the
     GEMV 28)."""
-    m = x2.shape[0]
-    return m <= _lib.GEMV_MAX_ROWS and (_approx(m, mul1) or
-                                        (x2.is_cuda and E.captures_without_prefill_workspace(x2)))
+    return (GEMV_APPROX != "" and _approx(x2.shape[0], mul1)) or (x2.is_cuda and E.captures_without_prefill_workspace(x2))
 
+
+def _gemv(m: int, x2: torch.Tensor, mul1: bool, k: int, width: int, K: int, widths: Optional[tuple] = None,
+          ldy: Optional[int] = None, held: bool = False) -> bool:
+    """gemv_rows(..., held or _hold) of a launch over the m rows x2, for the ops: no boundary lies below MID_MR or
+    above the GEMV's rows, and _hold only raises one, so it asks for no more than decides the call (an eager
+    call's host time: every question at every call took an MLP of 20 rows from 71.3 to 74.7 us, these 72.0)."""
+    if MR_MAX is not None:
+        return m <= MR_MAX
+    if m <= MID_MR:
+        return True
+    if m > _lib.GEMV_MAX_ROWS:
+        return False
+    if held or PREFILL_ROUTE == "recon" or GEMM_KERNEL or not _rd_serves(k, widths or (width,), K, ldy or width):
+        return m <= PREFILL_CROSSOVER.get((k, width), DEFAULT_MR)
+    if m <= _crossover(k, width, K):
+        return True
+    return m <= PREFILL_CROSSOVER.get((k, width), DEFAULT_MR) and _hold(x2, mul1)
 
 
 _wbuf: dict = {}
@@ -215,13 +225,11 @@ def _prep(x: torch.Tensor):
     return x2, k
 
 
-def _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y, gemv: Optional[bool] = None):
+def _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y, gemv: bool):
     """One group into y ([M, n] view, unit column stride, any row stride); gemv: the route chosen
-    by the caller for the launch this group belongs to (None: by this group's own shape)."""
+    by the caller for the launch this group belongs to."""
     M, k = x2.shape
     n = svh.shape[0]
-    if gemv is None:
-        gemv = _few(M) or gemv_rows(M, k, n, K, (n,), y.stride(0), _hold(x2, mul1))
     if gemv and _approx(M, mul1):
         rc = E.exl3_gemv_mr_approx(x2, trellis, y, suh, None, svh, K, GEMV_APPROX)
         if rc != 0:
@@ -263,7 +271,7 @@ def _linear(x: torch.Tensor, trellis: torch.Tensor, suh: torch.Tensor, svh: torc
     M = x2.shape[0]
     y = torch.empty((M, n), dtype=torch.float16, device=x.device)
     if M:
-        _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y)
+        _linear_into(x2, trellis, suh, svh, K, mcg, mul1, y, _gemv(M, x2, mul1, k, n, K))
     return _shaped(y, x)
 
 
@@ -296,20 +304,19 @@ def _linear_groups(x: torch.Tensor, trellis: list[torch.Tensor], suh: list[torch
     ng = len(trellis)
     if M == 0:                                        # every route: an empty batch launches nothing
         return x2.new_empty((*x.shape[:-1], sum(widths)), dtype=torch.float16)
-    y = torch.empty((M, sum(widths)), dtype=torch.float16, device=x.device)
+    n_all = sum(widths)
+    y = torch.empty((M, n_all), dtype=torch.float16, device=x.device)
     # runs of consecutive groups with equal K share one launch, each group written straight into
     # its row-strided column slice; each run takes the route of its own shape (EXL3_GATED=fused: gate and
     # up that of their one-launch form, so that both stay bitwise the same)
-    few = _few(M)
-    hold = few or _hold(x2, mul1) or (GATED_ROUTE == "fused" and ng == 2 and K[0] == K[1] and widths[0] == widths[1]
-                                     and M <= _lib.GEMV_FUSED_MAX_ROWS)
+    held = GATED_ROUTE == "fused" and ng == 2 and K[0] == K[1] and widths[0] == widths[1] and M <= _lib.GEMV_FUSED_MAX_ROWS
     i, n0 = 0, 0
     while i < ng:
         j = i + 1
         while j < ng and j - i < _lib.MAX_GROUPS and K[j] == K[i]:
             j += 1
         w = sum(widths[i:j])
-        gemv = few or gemv_rows(M, k, w, K[i], tuple(widths[i:j]), y.stride(0), hold)
+        gemv = _gemv(M, x2, mul1, k, w, K[i], tuple(widths[i:j]), n_all, held)
         if j == i + 1 or (gemv and _approx(M, mul1)) or \
                 (not gemv and PREFILL_ROUTE == "recon"):
             # one group, the approximate GEMV or the recon prefill: each group its own launch
@@ -402,7 +409,7 @@ def exl3_silu_mul_linear(gu: torch.Tensor, trellis: torch.Tensor, suh: torch.Ten
     if M == 0:
         return y.view(*gu.shape[:-1], n)
     approx = _approx(M, mul1)
-    gemv = _few(M) or gemv_rows(M, k, n, K, hold=_hold(g2, mul1))
+    gemv = _gemv(M, g2, mul1, k, n, K)
     if gemv and M <= _lib.GEMV_FUSED_MAX_ROWS and not approx:
         rc = E.exl3_gemv_silu_in(g2[:, :k], g2[:, k:], trellis, y, suh, None, svh, K, mcg, mul1)
         if rc != 0:

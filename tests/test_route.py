@@ -206,6 +206,25 @@ def test_capture_without_the_prefill_workspace(monkeypatch, m, gemv):
     assert ops.gemv_rows(m, k, n, hold=ops._hold(Input, True)) == (m <= 8)
 
 
+@pytest.mark.parametrize("knobs", [{}, {"MR_MAX": 16}, {"PREFILL_ROUTE": "recon"}, {"GEMM_KERNEL": "pc"}, {"GEMV_APPROX": "affine"}])
+@pytest.mark.parametrize("captures", [False, True])
+def test_the_ops_question_is_the_rule(monkeypatch, knobs, captures):
+    """_gemv, which leaves out what cannot decide a call, against gemv_rows with every question asked."""
+    for name, value in knobs.items():
+        monkeypatch.setattr(ops, name, value)
+    rec = _Mlp()
+    rec.captures_without_prefill_workspace = lambda x: captures
+    monkeypatch.setattr(ops, "E", rec)
+    shapes = CHECKPOINT + [(4096, 4096), (2048, 2048), (512, 512), (3200, 1024), (8192, 262144)]
+    for k, w in shapes:
+        for m in [*range(1, 66), 128, 2048]:
+            x = type("Rows", (), dict(shape=(m, k), is_cuda=True))
+            for K in (2, 8):
+                for held in (False, True):
+                    want = ops.gemv_rows(m, k, w, K, hold=held or ops._hold(x, True))
+                    assert ops._gemv(m, x, True, k, w, K, held=held) == want, (m, k, w, K, held)
+
+
 def test_launches_that_need_no_workspace_allocate_none(workspaces):
     def ws(m, k, widths, K=4, stream=5):
         return E._launch_workspace(CPU, stream, m, k, (ctypes.c_int * len(widths))(*widths), len(widths), K, sum(widths))
