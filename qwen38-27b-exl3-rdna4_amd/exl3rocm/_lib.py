@@ -98,5 +98,5 @@ def check(rc: int, what: str) -> int:
 
 
 def ptr_array(ptrs):
-    arr = (C.c_void_p * len(ptrs))(*ptrs)
-    return C.cast(arr, _pp), arr
+    """A host array of pointers, itself a `_pp` argument (a cast to one took an eager call 1.4 us each)."""
+    return (C.c_void_p * len(ptrs))(*ptrs)

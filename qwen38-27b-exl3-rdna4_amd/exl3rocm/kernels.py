@@ -308,9 +308,9 @@ def exl3_gemv_mr_grouped(A, B: Sequence[torch.Tensor], C, suh: Sequence[torch.Te
     st = _stream(A)
     ws = workspace(A.device, gemv_workspace_bytes(m, k, n, K, g), st)
     xr = _rot_scratch(A_had, A.device, g, m, k)
-    pt, _a = L.ptr_array([b.data_ptr() for b in B])
-    ps, _b = L.ptr_array([s.data_ptr() for s in suh])
-    pv, _c = L.ptr_array([s.data_ptr() for s in svh])
+    pt = L.ptr_array([b.data_ptr() for b in B])
+    ps = L.ptr_array([s.data_ptr() for s in suh])
+    pv = L.ptr_array([s.data_ptr() for s in svh])
     return L.check(L.lib().exl3_gemv_mr_grouped(x2.data_ptr(), x2.stride(0) if m > 1 else k, pt, C.data_ptr(),
                                                 _ldy(C, g * n), ps, xr.data_ptr() if xr is not None else None, pv,
                                                 g, m, k, n, K, *_cb_flags(mcg, mul1),
@@ -332,9 +332,9 @@ def exl3_gemv_mr_grouped_widths(A, B: Sequence[torch.Tensor], C, suh: Sequence[t
     st = _stream(A)
     ws = workspace(A.device, int(L.lib().exl3_gemv_workspace_size_widths(m, k, wa, g)), st)
     xr = _rot_scratch(A_had, A.device, g, m, k)
-    pt, _a = L.ptr_array([b.data_ptr() for b in B])
-    ps, _b = L.ptr_array([s.data_ptr() for s in suh])
-    pv, _c = L.ptr_array([s.data_ptr() for s in svh])
+    pt = L.ptr_array([b.data_ptr() for b in B])
+    ps = L.ptr_array([s.data_ptr() for s in suh])
+    pv = L.ptr_array([s.data_ptr() for s in svh])
     return L.check(L.lib().exl3_gemv_mr_grouped_widths(x2.data_ptr(), x2.stride(0) if m > 1 else k, pt, C.data_ptr(),
                                                        _ldy(C, sum(widths)), ps,
                                                        xr.data_ptr() if xr is not None else None, pv, wa, g, m, k, K,
@@ -355,9 +355,9 @@ def exl3_gemv_silu_mul(A, B: Sequence[torch.Tensor], C, suh: Sequence[torch.Tens
     st = _stream(A)
     ws = workspace(A.device, gemv_workspace_bytes(m, k, n, K, 2), st)
     xr = _rot_scratch(None, A.device, 2, m, k)
-    pt, _a = L.ptr_array([b.data_ptr() for b in B])
-    ps, _b = L.ptr_array([s.data_ptr() for s in suh])
-    pv, _c = L.ptr_array([s.data_ptr() for s in svh])
+    pt = L.ptr_array([b.data_ptr() for b in B])
+    ps = L.ptr_array([s.data_ptr() for s in suh])
+    pv = L.ptr_array([s.data_ptr() for s in svh])
     return L.check(L.lib().exl3_gemv_silu_mul(x2.data_ptr(), x2.stride(0) if m > 1 else k, pt, C.data_ptr(),
                                               _ldy(C, n), ps, xr.data_ptr() if xr is not None else None, pv, m, k, n,
                                               K, *_cb_flags(mcg, mul1), ws.data_ptr(),
@@ -481,9 +481,9 @@ def exl3_gemm_trellis_grouped(A, B: Sequence[torch.Tensor], C, suh: Sequence[tor
     _need(xh.numel() >= g * m * k and xh.dtype == torch.float16 and xh.is_contiguous(),
           "grouped gemm: xh scratch [groups, m, k] fp16")
     wa = (C_int * g)(*widths)
-    pt, _a = L.ptr_array([b.data_ptr() for b in B])
-    ps, _b = L.ptr_array([s.data_ptr() for s in suh])
-    pv, _c = L.ptr_array([s.data_ptr() for s in svh])
+    pt = L.ptr_array([b.data_ptr() for b in B])
+    ps = L.ptr_array([s.data_ptr() for s in suh])
+    pv = L.ptr_array([s.data_ptr() for s in svh])
     st = _stream(A)
     ldy = _ldy(C, sum(widths))
     ws = _launch_workspace(A.device, st, m, k, wa, g, K, ldy)
