@@ -598,9 +598,9 @@ def small_batch(torch, sets, ms=(1, 2, 4, 8, 12, 16, 17, 20, 24, 28, 32, 33, 36,
                 reps=32):
     """Configuration 3: gate (5120 -> 17408), down (17408 -> 5120) and the grouped gate/up launch
     (5120 -> 2 x 17408) at M from 1 to 256, heavy-tail activations.  Per M: the op (its route: the
-    fused GEMV up to the measured crossover b of the launch's shape, the prefill GEMM above), the
-    GEMV (<= 64 rows) and the prefill GEMM called directly, and the GEMM without a workspace (its
-    tiles unsplit, the plan's comparison) at M in {4, ..., 256}.  Also b, the step at the route
+    fused GEMV up to the measured crossover b of the launch's shape, a GEMM above: up to 128 rows the
+    register-decode GEMM, then the prefill GEMM), the GEMV (<= 64 rows) and the GEMM route called
+    directly, and the prefill GEMM without a workspace (its tiles unsplit, the plan's comparison) at M in {4, ..., 256}.  Also b, the step at the route
     boundary op(b + 1) / op(b) - 1, the op's worst ratio to the faster route over M <= 64, and the
     smallest M at which the GEMM beats the GEMV.  Mean duration per call from a graph of `reps`
     calls over the weight copies (HIP events on the replay stream): the median of three blocks of
@@ -816,8 +816,8 @@ def main() -> int:
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--traffic-probe", action="store_true", help="only the dispatches the PMC traffic passes read")
     ap.add_argument("--config3-only", action="store_true",
-                    help="only the configuration-3 section (the GEMV at small M, the prefill GEMM split and "
-                         "unsplit at M = 4-256; what its kernel-trace profile reads); prints its dict")
+                    help="only the configuration-3 section (the GEMV at small M, the GEMM route and the prefill "
+                         "GEMM unsplit at M = 4-256; what its kernel-trace profile reads); prints its dict")
     ap.add_argument("--timeline", action="store_true",
                     help="only the per-workgroup phase timeline of each configuration-1 GEMV launch (loads the "
                          "tracing library exl3rocm/libexl3_mi355x_timeline.so: build_ext.py --timeline)")

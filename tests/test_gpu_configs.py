@@ -390,7 +390,7 @@ ROUTE_CASES = [(6144, (5120,), 4), (5120, (17408,), 4), (5120, (17408, 17408), 4
 @pytest.mark.parametrize("k,widths,bits", ROUTE_CASES)
 def test_routing_follows_the_measured_crossover(k, widths, bits):
     """linear / linear_groups at the measured crossover b of the launch's shape and at b + 1: the
-    (grouped) GEMV launch at b rows and the grouped prefill GEMM at b + 1, bitwise; the first and
+    (grouped) GEMV launch at b rows and the grouped GEMM entry point at b + 1, bitwise; the first and
     last rows of both against the oracle."""
     if ops.PREFILL_ROUTE != "fused":
         pytest.skip("EXL3_PREFILL selects the reconstruct + GEMM route above the boundary")
